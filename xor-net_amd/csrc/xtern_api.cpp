@@ -314,25 +314,19 @@ int run_product(const xt_weights* const* ws, int n, const int8_t* q, int ldq, co
     a.nch = (int)ws[0]->nch;
     a.cps = (a.nch + cfg.splitk - 1) / cfg.splitk;
     const int64_t gy = (M + 16 * cfg.mb - 1) / (16 * cfg.mb);
-    if (gy > 65535) return fail(XT_ERR_UNSUPPORTED, "M too large for one launch");
+    // (rows per launch: 65535 blocks of 32 tokens up to 18 Pack4 or 8 Pack5
+    // chunks of K, of 16 tokens beyond)
+    const int64_t block = a.nch <= (fmt == XT_PACK5 ? 8 : 18) ? 32 : 16;
+    if (M > 65535 * block || (cfg.kind != 4 && gy > 65535)) return fail(XT_ERR_UNSUPPORTED, "M too large for one launch");
     if (cfg.kind == 2) {
         a.rg = cfg.nb;
         hipError_t e = xt::launch_gemv(fmt, a, tiles, cfg.waves, s);
         if (e != hipSuccess) return hip_fail(e, "ternary GEMV launch");
         return XT_OK;
     }
-    if (cfg.kind == 1 || cfg.kind == 3) {
-        if (cfg.splitk > 1) {
-            void* wsp = nullptr;
-            size_t region = 0;
-            const size_t pbytes = align_up((size_t)cfg.splitk * M * cols * sizeof(int32_t), 256);
-            if (int rc = splitk_workspace(s, 0, pbytes, &wsp, &region, sc)) return rc;
-            a.part = reinterpret_cast<int32_t*>(static_cast<char*>(wsp) + region);
-        }
-        a.ldp = cols;
-        hipError_t e = cfg.kind == 3 ? xt::launch_gemm32(a, tiles, cfg.splitk, s)
-                                     : xt::launch_gemm(fmt, a, tiles, cfg.splitk, s);
-        if (e != hipSuccess) return hip_fail(e, "ternary GEMM launch");
+    if (cfg.kind == 4) {
+        hipError_t e = xt::launch_gemmw(fmt, cfg.mb / 2, cfg.nb / 2 / cfg.waves, cfg.waves, a, tiles, s);
+        if (e != hipSuccess) return hip_fail(e, "prefill GEMM launch");
         return XT_OK;
     }
     if (cfg.splitk > 1) {
@@ -351,16 +345,6 @@ int run_product(const xt_weights* const* ws, int n, const int8_t* q, int ldq, co
     hipError_t e = xt::launch_mm(fmt, cfg, a, tiles, s);
     if (e != hipSuccess) return hip_fail(e, "ternary product launch");
     return XT_OK;
-}
-
-// Whether the product for M rows needs the quantiser's activation row sums:
-// only the Pack5 prefill GEMM multiplies codes with a caller row sum; the
-// other kernels decode signed weights or sum the rows themselves (measured:
-// computing them for the long-K kernel costs more in the quantiser than the
-// kernel's own extra MFMA per k-step saves).
-bool wants_rowsum(const xt_weights* w, int64_t M) {
-    if (xt::is_int_format(w->fmt) || w->fmt == XT_XORSPARSE_STREAM) return false;
-    return xt::choose_config(w->fmt, (int)M, 0, (int)w->nch, true).kind == 1;
 }
 
 int check_group(const xt_weights* const* ws, int n, const void* in, int64_t M, float* const* ys) {
@@ -385,22 +369,17 @@ int linear_q(const xt_weights* const* ws, int n, const int8_t* q, const float* i
     if (M == 0) return XT_OK;
     const int64_t K = ws[0]->K;
     const int64_t kpad = ws[0]->nch * xt::chunk_cols(ws[0]->fmt);
-    const bool need_rowsum = wants_rowsum(ws[0], M);
     const bool direct = (kpad == K) && ((((uintptr_t)q) & 15) == 0);
-    if (direct && user_rowsum)
-        return run_product(ws, n, q, (int)K, inv, user_rowsum, M, ys, acc, s);
-    if (direct && !need_rowsum)
-        return run_product(ws, n, q, (int)K, inv, nullptr, M, ys, acc, s);
-    // Padded copy and/or row sums in the workspace.
-    const size_t qbytes = direct ? 0 : align_up((size_t)M * kpad, 256);
+    if (direct) return run_product(ws, n, q, (int)K, inv, user_rowsum, M, ys, acc, s);
+    // Padded copy and row sums in the workspace.
+    const size_t qbytes = align_up((size_t)M * kpad, 256);
     void* wsp = nullptr;
     if (int rc = workspace(s, qbytes + align_up((size_t)M * 4, 256), &wsp)) return rc;
-    int8_t* qpad = direct ? nullptr : static_cast<int8_t*>(wsp);
+    int8_t* qpad = static_cast<int8_t*>(wsp);
     int32_t* rowsum = reinterpret_cast<int32_t*>(static_cast<char*>(wsp) + qbytes);
     hipError_t e = xt::launch_rowsum(q, K, (int)M, (int)K, qpad, (int)kpad, rowsum, s);
     if (e != hipSuccess) return hip_fail(e, "row-sum launch");
-    return run_product(ws, n, direct ? q : qpad, (int)(direct ? K : kpad), inv, rowsum, M, ys, acc,
-                       s);
+    return run_product(ws, n, qpad, (int)kpad, inv, rowsum, M, ys, acc, s);
 }
 
 // Small inputs on the GEMV: the kernel quantises the f32 rows itself (no
@@ -494,12 +473,9 @@ int linear_f32(const xt_weights* const* ws, int n, const float* x, int64_t M, fl
     if (int rc = workspace(s, qbytes + 2 * fbytes, &wsp, 0, sc)) return rc;
     int8_t* q = static_cast<int8_t*>(wsp);
     float* inv = reinterpret_cast<float*>(static_cast<char*>(wsp) + qbytes);
-    int32_t* rowsum = wants_rowsum(ws[0], M)
-                          ? reinterpret_cast<int32_t*>(static_cast<char*>(wsp) + qbytes + fbytes)
-                          : nullptr;
-    hipError_t e = xt::launch_quantize(x, K, (int)M, (int)K, q, (int)kpad, inv, rowsum, mode, s);
+    hipError_t e = xt::launch_quantize(x, K, (int)M, (int)K, q, (int)kpad, inv, nullptr, mode, s);
     if (e != hipSuccess) return hip_fail(e, "quantize launch");
-    return run_product(ws, n, q, (int)kpad, inv, rowsum, M, ys, nullptr, s, sc);
+    return run_product(ws, n, q, (int)kpad, inv, nullptr, M, ys, nullptr, s, sc);
 }
 
 int launch_mid(const xt::MidArgs& a, int64_t M, hipStream_t s) {
@@ -545,13 +521,12 @@ int mlp_run(const xt_weights* gate, const xt_weights* up, const xt_weights* down
     const size_t qb = align_up((size_t)M * kpad, 256);
     const size_t sb = align_up((size_t)M * 4, 256);
     void* wsp = nullptr;
-    if (int rc = workspace(s, 2 * fb + qb + 2 * sb, &wsp, 2)) return rc;
+    if (int rc = workspace(s, 2 * fb + qb + sb, &wsp, 2)) return rc;
     char* base = static_cast<char*>(wsp);
     float* g = reinterpret_cast<float*>(base);
     float* u = reinterpret_cast<float*>(base + fb);
     int8_t* qm = reinterpret_cast<int8_t*>(base + 2 * fb);
     float* invm = reinterpret_cast<float*>(base + 2 * fb + qb);
-    int32_t* rsm = reinterpret_cast<int32_t*>(base + 2 * fb + qb + sb);
     const xt_weights* gu[2] = {gate, up};
     float* gy[2] = {g, u};
     int rc = in_is_f32 ? linear_f32(gu, 2, static_cast<const float*>(in), M, gy, mode, s)
@@ -571,12 +546,10 @@ int mlp_run(const xt_weights* gate, const xt_weights* up, const xt_weights* down
     a.q = qm;
     a.ldq = (int)kpad;
     a.inv = invm;
-    // row sums of the requantised rows only for a down product that uses them
-    a.rowsum = wants_rowsum(down, M) ? rsm : nullptr;
     if ((rc = launch_mid(a, M, s))) return rc;
     float* ys[1] = {y};
     const xt_weights* dw[1] = {down};
-    return run_product(dw, 1, qm, (int)kpad, invm, a.rowsum, M, ys, nullptr, s);
+    return run_product(dw, 1, qm, (int)kpad, invm, nullptr, M, ys, nullptr, s);
 }
 
 }  // namespace

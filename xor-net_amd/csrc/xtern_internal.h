@@ -53,7 +53,7 @@ struct MMArgs {
     int ldq;
     int nch;                // chunks per row
     int cps;                // chunks per split-K slice (blockIdx.z)
-    int32_t* part;          // split-K partial sums [M][ldp], all zero between calls
+    int32_t* part;          // split-K partial sums, one plane [M][ldp] per slice
     int ldp;
     unsigned* cnt;          // split-K arrival counters, one per (x, y) tile, zero between calls
     // GEMV only: when x is set the kernel quantises the f32 rows x [M][ldx]
@@ -63,6 +63,7 @@ struct MMArgs {
     int K;
     int mode;
     int rg;                 // decode GEMV: 16-row groups per workgroup (0 or 1: one)
+    int gx;                 // gemmw_kernel: workgroup columns (set by its launcher)
 };
 // GEMV with the quantiser fused when M * K is at most this (every workgroup
 // re-reads the f32 rows, so only for small inputs).  The staging-free GEMV
@@ -91,8 +92,8 @@ hipError_t launch_gstream(int fmt, const GStreamArgs& a, int grid, int d, hipStr
 struct MMConfig {
     int mb, nb, waves, pf;  // tokens per WG = 16*mb, rows per WG = 16*nb
     int splitk;             // workgroups along K (blockIdx.z)
-    int kind = 0;           // 0 mm_kernel, 1 prefill GEMM, 2 decode GEMV (waves used),
-                            // 3 prefill GEMM on 32x32x32 MFMA (Pack4 tiles)
+    int kind = 0;           // 0 mm_kernel, 2 decode GEMV (waves used), 4 gemmw_kernel
+                            // (mb = 2 mw, nb = 2 nw waves)
 };
 
 // Kernel launchers (xtern_kernels.hip).  Return the hipError_t of the launch.
@@ -103,15 +104,11 @@ hipError_t launch_rowsum(const int8_t* qin, int64_t ldin, int M, int K, int8_t* 
 hipError_t launch_mm(int fmt, const MMConfig& cfg, const MMArgs& a, int ntiles_total,
                      hipStream_t s);
 MMConfig choose_config(int fmt, int M, int ntiles_nb1, int nch, bool have_rowsum);
-// Prefill GEMM (M > 16, row sums required): 32 tokens x 128 rows per
-// workgroup, at most gemm_ncmax(fmt) chunks per split-K slice.
-int gemm_ncmax(int fmt);
-hipError_t launch_gemm(int fmt, const MMArgs& a, int ntiles, int splitk, hipStream_t s);
-// Prefill GEMM on 32x32x32 MFMA (Pack4 tiles, M > 16, row sums required):
-// 32 tokens x 128 rows per workgroup, at most gemm32_ncmax() chunks per slice.
-int gemm32_ncmax();
-int g32_splitk(int nch);
-hipError_t launch_gemm32(const MMArgs& a, int ntiles, int splitk, hipStream_t s);
+// Prefill GEMM for many rows (xtern_gemm.hip): 32 mw tokens x 32 nw output
+// rows per wave, w waves per workgroup, over all of K; ntiles counts
+// workgroup columns.
+bool gemmw_known(int fmt, int mw, int nw, int w);
+hipError_t launch_gemmw(int fmt, int mw, int nw, int w, const MMArgs& a, int ntiles, hipStream_t s);
 // Decode GEMV (M <= 16): 16 output rows per workgroup, activations in LDS.
 hipError_t launch_gemv(int fmt, const MMArgs& a, int ntiles, int waves, hipStream_t s);
 int gemv_ncw(int waves);

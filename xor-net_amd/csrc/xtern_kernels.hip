@@ -1347,648 +1347,17 @@ hipError_t launch_gemv(int fmt, const MMArgs& a, int ntiles, int waves, hipStrea
     return hipErrorInvalidValue;
 }
 
-// ---------------------------------------------------------------------------
-// Prefill GEMM (M > 16): one load round per workgroup
-// ---------------------------------------------------------------------------
-//
-// Workgroup (x, y, z): 32 tokens (y) x 128 output rows (x) over chunk slice z
-// of at most NCMAX chunks.  Its 8 waves are 4 row groups of 32 rows x 2
-// chunk groups (even / odd chunks of the slice).  At entry every thread
-// issues all of its loads: the activation slice (32 x slice bytes, coalesced
-// 16-byte pieces) goes to LDS in MFMA A-operand order
-// [chunk][step][token block][lane][16 B], and each wave pulls its own weights
-// (32 rows x its chunks) into registers.  After one barrier the waves run
-// 2 x 2 accumulator blocks of 16x16x64 i8 MFMAs, prefetching the next
-// k-step's A operands from LDS before issuing the current step's MFMAs (two
-// waves per SIMD hide the rest).  The two chunk groups are added through LDS.
-// gridDim.z == 1 writes y; otherwise the slice's code-domain partial sums go
-// to plane z of `part` and gemm_reduce_kernel finishes.
-template <int FMT, int NCMAX, int KG>
-__global__ __launch_bounds__(256 * KG) void gemm_kernel(const MMArgs a) {
-    constexpr int STEPS = (FMT == XT_PACK5) ? 5 : 4;
-    constexpr int CH = STEPS * 64;
-    constexpr int SEGS = CH / 16;       // 16-byte pieces per token per chunk
-    constexpr int MB = 2;               // token blocks of 16
-    constexpr int NBW = 2;              // output-row blocks of 16 per wave
-    constexpr int NCW = (NCMAX + KG - 1) / KG;  // chunks per wave
-    constexpr int NT = 256 * KG;                 // threads
-    extern __shared__ __align__(16) uint8_t lds_a[];
-    __shared__ v4i red[KG - 1][4][MB * NBW][64];
-
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int ngrp = wave & 3;          // row group of 32 rows
-    const int kgrp = wave >> 2;         // chunks kgrp, kgrp + KG, ...
-    const int g = lane >> 4;
-    const int j = lane & 15;
-
-    // Logical tile: token blocks (y) fastest, so the token blocks that read the
-    // same weight rows sit on one XCD and share its L2.
-    const int gx = gridDim.x, gy = gridDim.y;
-    const int lin = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
-    const int t = xcd_remap(lin, gx * gy * gridDim.z);
-    const int by = t % gy;
-    const int bx = (t / gy) % gx;
-    const int bz = t / (gx * gy);
-    const ProjView pv = select_proj(proj_bounds(), bx);
-    const uint8_t* tiles = pv.tiles;
-    const float* ws = pv.ws;
-    float* y = pv.y;
-    int32_t* accout = pv.acc;
-    const int N = pv.N;
-    const int tile0 = pv.tile0;
-    const int col0 = pv.col0;
-    const int NG = (N + 15) >> 4;
-    const int M = a.M;
-    const int mbase = by * 32;
-    const int nch = a.nch;
-    const int cbeg = bz * a.cps;
-    const int nc = min(nch - cbeg, a.cps);  // chunks in this slice (<= NCMAX)
-    const int gbase = (bx - tile0) * 8 + ngrp * NBW;  // first row group of this wave
-
-    // Weights of this wave: NBW row groups x its chunks, 16 bytes per lane each.
-    v4i wv[NCW][NBW];
-#pragma unroll
-    for (int u = 0; u < NCW; ++u)
-#pragma unroll
-        for (int nb = 0; nb < NBW; ++nb) {
-            const int cc = kgrp + KG * u;
-            const int G = gbase + nb;
-            wv[u][nb] = (cc < nc && G < NG)
-                            ? *reinterpret_cast<const v4i*>(tiles + ((size_t)(G * nch + cbeg + cc) * 64 + lane) * 16)
-                            : v4i{0, 0, 0, 0};
-        }
-
-    // Epilogue operands now, so no memory round trip is left after the MFMAs.
-    const bool split = gridDim.z > 1;
-    float wsc[NBW];
-#pragma unroll
-    for (int nb = 0; nb < NBW; ++nb) {
-        const int o = (gbase + nb) * 16 + j;
-        wsc[nb] = (!split && kgrp == 0 && o < N) ? ws[o] : 0.0f;
-    }
-    float invr[MB][4];
-    int rsr[MB][4];
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int i = mbase + mb * 16 + 4 * g + r;
-            const bool ok = !split && kgrp == 0 && i < M;
-            invr[mb][r] = ok ? a.inv[i] : 0.0f;
-            rsr[mb][r] = ok ? a.rowsum[i] : 0;
-        }
-
-    // Activation slice -> LDS, A-operand order.  Pieces are taken in LDS
-    // order (lane fastest), so the LDS stores are sequential; the global side
-    // reads 64-byte runs of 16 token rows.
-    // All of a thread's loads are issued before its first LDS store, so the
-    // slice costs one memory round trip, not one per piece.
-    const int pieces = 32 * nc * SEGS;
-    constexpr int PPT = (32 * NCMAX * SEGS + NT - 1) / NT;  // pieces per thread
-    v4i stage[PPT];
-#pragma unroll
-    for (int r = 0; r < PPT; ++r) {
-        const int p = threadIdx.x + r * NT;
-        const int ln = p & 63;
-        const int blk = p >> 6;                 // (cc * STEPS + st) * MB + mb
-        const int mb = blk % MB;
-        const int cs = blk / MB;                // cc * STEPS + st
-        const int row = mbase + mb * 16 + (ln & 15);
-        stage[r] = v4i{0, 0, 0, 0};
-        if (p < pieces && row < M)
-            stage[r] = ld_cached(a.q + (size_t)row * a.ldq + (size_t)cbeg * CH + cs * 64 + (ln >> 4) * 16);
-    }
-#pragma unroll
-    for (int r = 0; r < PPT; ++r) {
-        const int p = threadIdx.x + r * NT;
-        if (p < pieces) *reinterpret_cast<v4i*>(lds_a + ((size_t)p << 4)) = stage[r];
-    }
-    __syncthreads();
-
-    v4i acc[MB][NBW];
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-        for (int nb = 0; nb < NBW; ++nb) acc[mb][nb] = v4i{0, 0, 0, 0};
-
-    // A operands of k-step (u, s) of this wave; `nxt` is read one step ahead.
-    auto a_addr = [&](int u, int st, int mb) {
-        return lds_a + (((((kgrp + KG * u) * STEPS + st) * MB + mb) * 64 + lane) << 4);
-    };
-    v4i cur[MB], nxt[MB];
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-        cur[mb] = (kgrp < nc) ? *reinterpret_cast<const v4i*>(a_addr(0, 0, mb)) : v4i{0, 0, 0, 0};
-
-#pragma unroll
-    for (int u = 0; u < NCW; ++u) {
-        if (kgrp + KG * u < nc) {
-            int E[NBW][4], O[NBW][4];
-            if constexpr (FMT == XT_PACK5) {
-#pragma unroll
-                for (int nb = 0; nb < NBW; ++nb)
-#pragma unroll
-                    for (int d = 0; d < 4; ++d) {
-                        E[nb][d] = wv[u][nb][d] & 0x00ff00ff;
-                        O[nb][d] = ((unsigned)wv[u][nb][d] >> 8) & 0x00ff00ff;
-                    }
-            }
-#pragma unroll
-            for (int st = 0; st < STEPS; ++st) {
-                // prefetch the next k-step's operands
-                const int nu = (st + 1 < STEPS) ? u : u + 1;
-                const int ns = (st + 1 < STEPS) ? st + 1 : 0;
-                const bool have_next = (nu < NCW) && (kgrp + KG * nu < nc);
-#pragma unroll
-                for (int mb = 0; mb < MB; ++mb)
-                    nxt[mb] = have_next ? *reinterpret_cast<const v4i*>(a_addr(nu, ns, mb))
-                                        : v4i{0, 0, 0, 0};
-                v4i b[NBW];
-#pragma unroll
-                for (int nb = 0; nb < NBW; ++nb) {
-                    if constexpr (FMT == XT_PACK5) {
-#pragma unroll
-                        for (int d = 0; d < 4; ++d) {
-                            const int pE = E[nb][d] * 3, pO = O[nb][d] * 3;
-                            b[nb][d] = (int)__builtin_amdgcn_perm((unsigned)pO, (unsigned)pE, 0x07030501u);
-                            E[nb][d] = pE & 0x00ff00ff;
-                            O[nb][d] = pO & 0x00ff00ff;
-                        }
-                    } else {
-                        b[nb] = decode4(wv[u][nb][st]);
-                    }
-                }
-#pragma unroll
-                for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-                    for (int nb = 0; nb < NBW; ++nb) acc[mb][nb] = mfma(cur[mb], b[nb], acc[mb][nb]);
-#pragma unroll
-                for (int mb = 0; mb < MB; ++mb) cur[mb] = nxt[mb];
-            }
-        }
-    }
-
-    // Add the odd-chunk waves into the even-chunk waves, stage the 32 x 128
-    // tile in LDS (every wave is past its LDS operand reads at the first
-    // barrier), then all 512 threads write whole rows with 16-byte stores.
-    if (kgrp > 0) {
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-            for (int nb = 0; nb < NBW; ++nb) red[kgrp - 1][ngrp][mb * NBW + nb][lane] = acc[mb][nb];
-    }
-    __syncthreads();
-    float* ytile = reinterpret_cast<float*>(lds_a);            // [32][128]
-    int* dtile = reinterpret_cast<int*>(lds_a + 32 * 128 * 4);  // [32][128]
-    if (kgrp == 0) {
-#pragma unroll
-        for (int nb = 0; nb < NBW; ++nb) {
-            const int col = ngrp * 32 + nb * 16 + j;
-#pragma unroll
-            for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int row = mb * 16 + 4 * g + r;
-                    int v = acc[mb][nb][r];
-#pragma unroll
-                    for (int kk = 0; kk < KG - 1; ++kk) v += red[kk][ngrp][mb * NBW + nb][lane][r];
-                    if (split) {
-                        dtile[row * 128 + col] = v;
-                    } else {
-                        const int d = v - rsr[mb][r];
-                        // layers.rs:294 — (dot as f32 * inv_scale) * w_scale.
-                        ytile[row * 128 + col] = __fmul_rn(__fmul_rn((float)d, invr[mb][r]), wsc[nb]);
-                        dtile[row * 128 + col] = d;
-                    }
-                }
-        }
-    }
-    __syncthreads();
-    const int obase = (bx - tile0) * 128;
-    int32_t* plane = a.part + (size_t)bz * a.M * a.ldp;
-    const bool vec = (N & 3) == 0;
-    for (int idx = threadIdx.x; idx < 32 * 32; idx += NT) {
-        const int row = idx >> 5, c4 = (idx & 31) * 4;
-        const int i = mbase + row, o = obase + c4;
-        if (i >= M || o >= N) continue;
-        if (split) {
-            // planes have a padded stride (a multiple of 16 columns)
-            *reinterpret_cast<int4*>(plane + (size_t)i * a.ldp + col0 + o) =
-                *reinterpret_cast<const int4*>(dtile + row * 128 + c4);
-            continue;
-        }
-        if (vec && o + 3 < N) {
-            *reinterpret_cast<float4*>(y + (size_t)i * N + o) =
-                *reinterpret_cast<const float4*>(ytile + row * 128 + c4);
-            if (accout)
-                *reinterpret_cast<int4*>(accout + (size_t)i * N + o) =
-                    *reinterpret_cast<const int4*>(dtile + row * 128 + c4);
-        } else {
-            for (int e2 = 0; e2 < 4 && o + e2 < N; ++e2) {
-                y[(size_t)i * N + o + e2] = ytile[row * 128 + c4 + e2];
-                if (accout) accout[(size_t)i * N + o + e2] = dtile[row * 128 + c4 + e2];
-            }
-        }
-    }
-}
-
-// Sum the split-K planes of every projection and apply the epilogue.
-// One thread per (token, workspace column).
-__global__ __launch_bounds__(256) void gemm_reduce_kernel(const MMArgs a, int nsplit) {
-    const int i = blockIdx.y;
-    const int col = blockIdx.x * 256 + threadIdx.x;
-    if (col >= a.ldp || i >= a.M) return;
-    int p = 0;
-#pragma unroll
-    for (int q = 1; q < 4; ++q)
-        if (q < a.nproj && col >= a.proj[q].col0) p = q;
-    const Proj& pr = a.proj[p];
-    const int o = col - pr.col0;
-    if (o >= pr.N) return;
-    const size_t plane_sz = (size_t)a.M * a.ldp;
-    int tot = 0;
-    for (int z = 0; z < nsplit; ++z) tot += a.part[z * plane_sz + (size_t)i * a.ldp + col];
-    const int d = tot - (a.rowsum ? a.rowsum[i] : 0);  // signed-decode kernels pass none
-    pr.y[(size_t)i * pr.N + o] = __fmul_rn(__fmul_rn((float)d, a.inv[i]), pr.ws[o]);
-    if (pr.acc) pr.acc[(size_t)i * pr.N + o] = d;
-}
-
-int gemm_ncmax(int fmt) { return fmt == XT_PACK5 ? 8 : 10; }
-
-hipError_t launch_gemm(int fmt, const MMArgs& a, int ntiles, int splitk, hipStream_t s) {
-    const dim3 grid(ntiles, (a.M + 31) / 32, splitk);
-    const int ch = fmt == XT_PACK5 ? 320 : 256;
-    size_t lds = (size_t)a.cps * ch * 32;
-    if (lds < 32 * 128 * 8) lds = 32 * 128 * 8;  // the staged output tile
-#ifndef XT_GEMM_KG
-#define XT_GEMM_KG 4
-#endif
-    constexpr int KG = XT_GEMM_KG;
-    if (fmt == XT_PACK5)
-        hipLaunchKernelGGL((gemm_kernel<XT_PACK5, 8, KG>), grid, dim3(256 * KG), lds, s, a);
-    else
-        hipLaunchKernelGGL((gemm_kernel<XT_PACK4, 10, KG>), grid, dim3(256 * KG), lds, s, a);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || splitk == 1) return e;
-    const dim3 rgrid((a.ldp + 255) / 256, a.M);
-    hipLaunchKernelGGL(gemm_reduce_kernel, rgrid, dim3(256), 0, s, a, splitk);
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
-// Prefill GEMM on v_mfma_i32_32x32x32_i8 (Pack4 / XorSparse tiles, M > 16)
-// ---------------------------------------------------------------------------
-//
-// The 32x32x32 i8 MFMA runs at twice the rate of 16x16x64 on gfx950 (about
-// 4.1 vs 2.6 POP/s measured on MI355X), so this kernel computes 32-token x
-// 32-row blocks.  Workgroup (x, y, z): 32 tokens (y) x 128 output rows (x)
-// over chunk slice z.  Its eight MFMA waves are 4 row blocks (n) x 2 column
-// halves (L) of every 256-column chunk.
-//
-// Operands.  B (weights) lane 32h + r holds output row r of the wave's 32
-// rows: tile G = 2n + r/16 of the block, tile lane 16(2L + h) + r%16, whose
-// dword s holds columns 64s + 32L + 16h .. +15.  One 16-byte tile slot per
-// lane and chunk therefore gives four k-steps (s = 0..3) of the wave's half
-// L.  A (activations) lane 32h + r' holds the same 16 columns of token r'.
-// The MFMA pairs byte b of A with byte b of B in lanes of equal h, so only
-// the pairing has to match, not any particular column order.
-typedef int v16i __attribute__((ext_vector_type(16)));
-
-__device__ __forceinline__ v16i mfma32(v4i a, v4i b, v16i c) {
-    return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
-}
-
-// 16 bytes per lane from global memory straight into LDS; the wave's 64
-// lanes fill 1 KiB at `wave_lds` in lane order.
-__device__ __forceinline__ void load_lds16(const void* g, uint8_t* wave_lds) {
-#if __HIP_DEVICE_COMPILE__
-    __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)wave_lds, 16, 0, 0);
-#endif
-}
-
-// s_waitcnt with only the vector-memory counter constrained (gfx9 encoding:
-// vmcnt bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8).
-// `vm` must fold to a constant (it is called from fully unrolled loops).
-#define XT_VMCNT_IMM(V) (((V) & 15) | (((V) >> 4) << 14) | (7 << 4) | (15 << 8))
-__device__ __forceinline__ void wait_vmcnt(int vm) {
-    switch (vm) {
-#define XT_W4(B) case B: __builtin_amdgcn_s_waitcnt(XT_VMCNT_IMM(B)); break;    \
-                 case B + 1: __builtin_amdgcn_s_waitcnt(XT_VMCNT_IMM(B + 1)); break; \
-                 case B + 2: __builtin_amdgcn_s_waitcnt(XT_VMCNT_IMM(B + 2)); break; \
-                 case B + 3: __builtin_amdgcn_s_waitcnt(XT_VMCNT_IMM(B + 3)); break;
-        XT_W4(0) XT_W4(4) XT_W4(8) XT_W4(12) XT_W4(16) XT_W4(20) XT_W4(24) XT_W4(28)
-        XT_W4(32) XT_W4(36) XT_W4(40) XT_W4(44) XT_W4(48) XT_W4(52) XT_W4(56) XT_W4(60)
-#undef XT_W4
-        default: __builtin_amdgcn_s_waitcnt(XT_VMCNT_IMM(0)); break;
-    }
-}
-
-// 32-bit LDS address of a pointer into shared memory.
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
-}
-// ds_read_b128 whose completion the caller waits for with lgkm_wait4.
-__device__ __forceinline__ v4i ds_read16(uint32_t addr) {
-    v4i v;
-    __asm__ volatile("ds_read_b128 %0, %1" : "=v"(v) : "v"(addr));
-    return v;
-}
-// Wait for all LDS reads; the operands tie the wait to the values read.
-__device__ __forceinline__ void lgkm_wait4(v4i& a, v4i& b, v4i& c, v4i& d) {
-    __asm__ volatile("s_waitcnt lgkmcnt(0)" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
-}
-
-
-// ---------------------------------------------------------------------------
-// Prefill GEMM, warp-specialised: loader waves stream chunks into LDS while
-// eight MFMA waves consume them
-// ---------------------------------------------------------------------------
-//
-// Measured on MI355X, one workgroup per CU pulls only ~33-50 bytes per clock
-// from L2, so the 160 KiB a 32-token x 128-row tile needs over K = 2560 take
-// ~2 us -- as long as its MFMA work -- and a wave that issues its own loads
-// stalls at issue until the memory pipeline drains.  Here four loader waves
-// issue every load as a direct-to-LDS copy (no registers), chunk by chunk,
-// and signal each landed chunk with a workgroup barrier; the eight MFMA waves
-// (operands as above, both read from LDS) compute chunk c while later chunks
-// are still in flight.  Slot c of LDS holds chunk c: 8 KiB of activations
-// (token row t at 256 t, 16-byte piece p in slot p ^ (t & 15), so that 16
-// tokens reading one piece hit 16 distinct bank groups) then the 8 weight
-// tiles of the block (1 KiB each, as in memory).  The loaders keep
-// kG32sAhead chunks in flight before they start signalling.  The two halves
-// L are added through LDS, the 32 x 128 code-domain tile is staged in LDS
-// and written as whole 16-byte row pieces.  With gridDim.z > 1 the slice's
-// code-domain sums go to plane z of `part` and gemm_reduce_kernel finishes.
-constexpr int kG32sSlot = 8192;
-// First LDS slot of the epilogue's exchange (2 slots) and output tile (2).
-__host__ __device__ constexpr int g32s_xch_slot(int ncmax) { return ncmax >= 3 ? 0 : ncmax; }
-#ifndef XT_G32S_AHEAD
-#define XT_G32S_AHEAD 4
-#endif
-constexpr int kG32sAhead = XT_G32S_AHEAD;
-
-template <int NCMAX>
-__global__ __launch_bounds__(768) void gemm32s_kernel(const MMArgs a) {
-    constexpr int CH = 256;
-    extern __shared__ __align__(16) uint8_t lds[];
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-
-    const ProjBounds pb = proj_bounds();
-    const int gx = gridDim.x, gy = gridDim.y, gz = gridDim.z;
-    const int M = a.M;
-    const int nch = a.nch;
-    const int cps = a.cps;
-    // (the bounds are consumed here, so their loads join the grid-size round
-    // instead of being sunk to their first use after it)
-    asm volatile("" ::"s"(pb.np), "s"(pb.t0), "s"(pb.t1), "s"(pb.t2), "s"(pb.t3), "s"(gx), "s"(gy), "s"(gz));
-    __builtin_amdgcn_sched_barrier(0);  // one round of argument loads
-    const int lin = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
-    const int t = xcd_remap(lin, gx * gy * gz);
-    const int by = t % gy;
-    const int bx = (t / gy) % gx;
-    const int bz = t / (gx * gy);
-    const ProjView pv = select_proj(pb, bx);
-    const int N = pv.N;
-    const int NG = (N + 15) >> 4;
-    const int mbase = by * 32;
-    const int cbeg = bz * cps;
-    const int nc = min(nch - cbeg, cps);  // chunks of this slice, 1..NCMAX
-
-    // The gy token blocks that share the weights start at different quarters
-    // of the slice (different HBM lines in flight; integer sums do not depend
-    // on the order).  Chunk c of the loop is slice chunk chunk_at(c); chunks
-    // past the slice re-read its last chunk and count as code 0.
-    const int rot = ((by & 3) * nc) >> 2;
-    auto chunk_at = [&](int c) {
-        const int cr = c + rot;
-        return c < nc ? (cr >= nc ? cr - nc : cr) : nc - 1;
-    };
-
-    if (wave >= 8) {
-        // Loader wave lw copies activation rows 8 lw .. 8 lw + 7 of every
-        // chunk (two 1 KiB direct-to-LDS copies), so each chunk's vmcnt is a
-        // compile-time number, and signals landed chunks with barriers.
-        const int lw = wave - 8;
-        const int8_t* as[2];
-#pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
-            const int tk = 4 * (2 * lw + jj) + (lane >> 4);
-            const int trow = min(mbase + tk, M - 1);
-            as[jj] = a.q + (size_t)trow * a.ldq + (size_t)cbeg * CH + ((lane & 15) ^ (tk & 15)) * 16;
-        }
-        constexpr int D = kG32sAhead < NCMAX ? kG32sAhead : NCMAX;
-#pragma unroll
-        for (int c = 0; c < NCMAX; ++c) {
-            const int cc = chunk_at(c);
-            uint8_t* slot = lds + c * kG32sSlot;
-            load_lds16(as[0] + cc * CH, slot + (2 * lw) * 1024);
-            load_lds16(as[1] + cc * CH, slot + (2 * lw + 1) * 1024);
-            if (c >= D - 1) {  // chunk c - D + 1 has landed
-                wait_vmcnt(2 * (D - 1));
-                __builtin_amdgcn_s_barrier();
-            }
-        }
-#pragma unroll
-        for (int c = NCMAX - D + 1; c < NCMAX; ++c) {
-            wait_vmcnt(2 * (NCMAX - 1 - c));
-            __builtin_amdgcn_s_barrier();
-        }
-        __builtin_amdgcn_s_barrier();  // the MFMA waves' exchange
-        __builtin_amdgcn_s_barrier();  // and output staging barriers
-        return;
-    }
-
-    const int n = wave & 3;
-    const int L = wave >> 2;
-    const int h = lane >> 5;
-    const int r = lane & 31;
-    const bool split = gz > 1;
-
-    // Output phase operands, loaded now: thread t writes tokens t/32 and
-    // t/32 + 16 of the tile, columns 4 (t % 32) .. +3.
-    const int srow = threadIdx.x >> 5;
-    const int sc4 = (threadIdx.x & 31) * 4;
-    const int ob = (bx - pv.tile0) * 128;
-    float sinv[2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u) sinv[u] = a.inv[min(mbase + srow + 16 * u, M - 1)];
-    float sws[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) sws[e] = pv.ws[min(ob + sc4 + e, N - 1)];
-
-    // This wave's weights: its 16-byte tile slot of every chunk, loaded into
-    // registers kG32sAhead chunks ahead of use.
-    const int G = min((bx - pv.tile0) * 8 + 2 * n + (r >> 4), NG - 1);
-    const uint8_t* wsrc = pv.tiles + ((size_t)(G * nch + cbeg) * 64 + 16 * (2 * L + h) + (r & 15)) * 16;
-    constexpr int DW = kG32sAhead < NCMAX ? kG32sAhead : NCMAX;
-    v4i wv[NCMAX];
-#pragma unroll
-    for (int c = 0; c < DW; ++c)
-        wv[c] = *reinterpret_cast<const v4i*>(wsrc + (size_t)chunk_at(c) * kTileBytes);
-
-    // Software-pipelined by one chunk: after the barrier that says chunk
-    // c + 1 has landed, the wave reads its A fragments while chunk c's four
-    // MFMAs (one accumulator per k-step, so none waits for another) run.
-    const uint32_t abase = lds_addr(lds) + r * CH;
-    auto read_a = [&](int c, v4i* av) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const int p = 4 * s + 2 * L + h;
-            av[s] = ds_read16(abase + c * kG32sSlot + ((p ^ (r & 15)) << 4));
-        }
-        lgkm_wait4(av[0], av[1], av[2], av[3]);
-    };
-    v16i acc[4];
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int k = 0; k < 16; ++k) acc[s][k] = 0;
-    v4i acur[4];
-    __syncthreads();  // chunk 0 has landed
-    read_a(0, acur);
-#pragma unroll
-    for (int c = 0; c < NCMAX; ++c) {
-        if (c + DW < NCMAX)
-            wv[c + DW] = *reinterpret_cast<const v4i*>(wsrc + (size_t)chunk_at(c + DW) * kTileBytes);
-        // chunks past the slice: code 1 everywhere, i.e. weight 0
-        const v4i bv = (c < nc) ? wv[c] : v4i{0x55555555, 0x55555555, 0x55555555, 0x55555555};
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            v4i b = decode4(bv[s]);
-#pragma unroll
-            for (int d = 0; d < 4; ++d) b[d] = signed_codes(b[d]);
-            acc[s] = mfma32(acur[s], b, acc[s]);
-        }
-        if (c + 1 < NCMAX) {
-            __syncthreads();  // chunk c + 1 has landed
-            read_a(c + 1, acur);
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < 16; ++k) acc[0][k] += acc[1][k] + acc[2][k] + acc[3][k];
-
-    // Add the halves L through LDS, in slots 0-1 when every wave is past
-    // their reads (their chunks completed before the last chunk's barrier),
-    // else after the chunk slots.  Entry [L][n][k][lane] carries registers
-    // 8(1 - L) + k for the other wave of the pair.
-    int32_t* xch = reinterpret_cast<int32_t*>(lds + g32s_xch_slot(NCMAX) * kG32sSlot);
-    int keep[8];
-    if (L == 0) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            xch[((0 * 4 + n) * 8 + k) * 64 + lane] = acc[0][8 + k];
-            keep[k] = acc[0][k];
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            xch[((1 * 4 + n) * 8 + k) * 64 + lane] = acc[0][k];
-            keep[k] = acc[0][8 + k];
-        }
-    }
-    __syncthreads();
-    // Code-domain sums of the 32 x 128 tile -> LDS (slot 1), then whole rows.
-    int32_t* dtile = reinterpret_cast<int32_t*>(xch + 4096);  // [32][128], two slots on
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const int il = 8 * (2 * L + (k >> 2)) + 4 * h + (k & 3);
-        dtile[il * 128 + 32 * n + r] = keep[k] + xch[(((1 - L) * 4 + n) * 8 + k) * 64 + lane];
-    }
-    __syncthreads();
-    const bool vec = (N & 3) == 0;
-    int32_t* plane = a.part + (size_t)bz * a.M * a.ldp;
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-        const int il = srow + 16 * u;
-        const int i = mbase + il;
-        const int o = ob + sc4;
-        if (i >= M || o >= N) continue;
-        const v4i d4 = *reinterpret_cast<const v4i*>(dtile + il * 128 + sc4);
-        if (split) {
-            // planes have a padded stride (a multiple of 16 columns)
-            *reinterpret_cast<v4i*>(plane + (size_t)i * a.ldp + pv.col0 + o) = d4;
-            continue;
-        }
-        float yv[4];
-        v4i dv;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            dv[e] = d4[e];
-            // layers.rs:294 — (dot as f32 * inv_scale) * w_scale.
-            yv[e] = __fmul_rn(__fmul_rn((float)dv[e], sinv[u]), sws[e]);
-        }
-        if (vec) {
-            *reinterpret_cast<float4*>(pv.y + (size_t)i * N + o) = make_float4(yv[0], yv[1], yv[2], yv[3]);
-            if (pv.acc) *reinterpret_cast<v4i*>(pv.acc + (size_t)i * N + o) = dv;
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                if (o + e < N) {
-                    pv.y[(size_t)i * N + o + e] = yv[e];
-                    if (pv.acc) pv.acc[(size_t)i * N + o + e] = dv[e];
-                }
-            }
-        }
-    }
-}
-
-int gemm32s_ncmax() { return 18; }
-
-hipError_t launch_gemm32s(const MMArgs& a, int ntiles, int splitk, hipStream_t s) {
-    const dim3 grid(ntiles, (a.M + 31) / 32, splitk);
-    const int ncm = a.cps;
-    if (ncm < 1 || ncm > gemm32s_ncmax()) return hipErrorInvalidValue;
-    const int xs = g32s_xch_slot(ncm) + 4;
-    const size_t lds = (size_t)(ncm < xs ? xs : ncm) * kG32sSlot;
-    switch (ncm) {
-#define XT_G32S(V) \
-    case V: hipLaunchKernelGGL((gemm32s_kernel<V>), grid, dim3(768), lds, s, a); break;
-        XT_G32S(1) XT_G32S(2) XT_G32S(3) XT_G32S(4) XT_G32S(5) XT_G32S(6) XT_G32S(7)
-        XT_G32S(8) XT_G32S(9) XT_G32S(10) XT_G32S(11) XT_G32S(12) XT_G32S(13) XT_G32S(14)
-        XT_G32S(15) XT_G32S(16) XT_G32S(17) XT_G32S(18)
-#undef XT_G32S
-        default: return hipErrorInvalidValue;
-    }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || splitk == 1) return e;
-    const dim3 rgrid((a.ldp + 255) / 256, a.M);
-    hipLaunchKernelGGL(gemm_reduce_kernel, rgrid, dim3(256), 0, s, a, splitk);
-    return hipGetLastError();
-}
-
-// Fewest K slices whose chunks fit the LDS stage of the prefill GEMM.
-int gemm32_ncmax() { return gemm32s_ncmax(); }
-int g32_splitk(int nch) { return nch <= 0 ? 1 : (nch + gemm32_ncmax() - 1) / gemm32_ncmax(); }
-hipError_t launch_gemm32(const MMArgs& a, int ntiles, int splitk, hipStream_t s) {
-    return launch_gemm32s(a, ntiles, splitk, s);
-}
-
 // Compiled tile shapes, selectable by MMConfig.
 #define XT_MM_SHAPES(X)  \
     X(1, 1, 4, 4)        \
-    X(1, 1, 2, 8)        \
-    X(1, 1, 2, 4)        \
     X(1, 1, 8, 2)        \
-    X(1, 1, 4, 2)        \
     X(1, 2, 4, 4)        \
     X(1, 4, 4, 2)        \
-    X(2, 4, 4, 2)        \
-    X(2, 8, 4, 2)        \
-    X(4, 4, 4, 1)        \
-    X(4, 2, 4, 1)        \
-    X(1, 5, 4, 2)        \
-    X(1, 5, 8, 2)        \
     X(1, 4, 8, 2)        \
-    X(2, 5, 8, 2)        \
-    X(1, 5, 16, 1)       \
-    X(1, 5, 8, 1)        \
-    X(1, 5, 16, 2)       \
-    X(1, 10, 8, 2)       \
-    X(2, 8, 8, 2)        \
+    X(1, 5, 8, 2)        \
     X(1, 8, 8, 2)        \
-    X(4, 4, 8, 1)
+    X(1, 5, 16, 1)       \
+    X(2, 8, 4, 2)
 
 namespace {
 bool shape_known(const MMConfig& c, bool own) {
@@ -1999,13 +1368,20 @@ bool shape_known(const MMConfig& c, bool own) {
     return false;
 }
 
-// XTERN_CONFIG="mb,nb,waves,pf,splitk" forces one tile shape (for tuning).
+// XTERN_CONFIG="mb,nb,waves,pf,splitk" forces one tile shape (for tuning),
+// "g32,S" S slices of K over workgroups, "gw,mw,nw,waves" one shape of the
+// many-row GEMM, "gemv,W" the decode GEMV.
 bool env_config(MMConfig* c) {
     const char* e = getenv("XTERN_CONFIG");
     MMConfig f;
     if (e && sscanf(e, "g32,%d", &f.splitk) == 1 && f.splitk >= 1) {
-        f = MMConfig{2, 8, 8, 1, f.splitk};
-        f.kind = 3;
+        *c = MMConfig{1, 4, 4, 2, f.splitk};
+        return true;
+    }
+    int mw = 0, nw = 0, w = 0;
+    if (e && sscanf(e, "gw,%d,%d,%d", &mw, &nw, &w) == 3) {
+        f = MMConfig{2 * mw, 2 * nw * w, w, 1, 1};
+        f.kind = 4;
         *c = f;
         return true;
     }
@@ -2024,13 +1400,6 @@ bool env_config(MMConfig* c) {
 }
 }  // namespace
 
-// Default tile shapes (chosen by measurement on MI355X):
-//   M <= 16  the decode GEMV (activations in LDS, 16 waves) when the staged
-//            activations fit, else 16 rows per workgroup, 8 waves x 2 chunks;
-//   M > 16   the prefill GEMM (32 tokens x 128 rows) when K fits one LDS
-//            slice, else 16 tokens x 64 rows with 4 waves splitting K.
-// Split-K across workgroups (gridDim.z > 1) is only taken when forced: its
-// device-scope release/acquire costs more than it saves at these sizes.
 // Waves per workgroup of the Int8 / Int4 GEMV for row blocks of mb tokens.
 int int_gemv_waves(int fmt, int mb, int nch) {
     MMConfig c;
@@ -2041,6 +1410,67 @@ int int_gemv_waves(int fmt, int mb, int nch) {
     return (fmt == XT_INT4 && gemv_fits(fmt, mb, nch, 8, gemv_ncw(8))) ? 8 : 16;
 }
 
+namespace {
+// Shapes of a product with more than 16 rows, and what one workgroup of each
+// costs per chunk of K: `first` when it has its CU to itself, `rest` for each
+// further workgroup of the CU, `gap` once per further workgroup (microseconds;
+// `unit`: K is taken in rounds of so many chunks).  Fitted to launch-to-launch
+// times on MI355X over M = 20 .. 2048 and K, N = 512 .. 14336 (weights
+// streamed from memory); with a few launches more or less per CU the totals
+// are within about 15 % of the measured ones, and where two shapes come out
+// close they measure close.
+struct GemmShape {
+    int mb, nb, waves, pf, kind;
+    float first, rest, gap;
+    int unit;
+};
+// 16-token shapes (mm_kernel) win while every CU gets at most one of them;
+// then ever larger tiles of gemmw_kernel.  Examples, us (16 x 64 / 16 x 128 /
+// 32 x 128 / 64 x 128 / 64 x 256 / 128 x 256): 2560 -> 6912 at M = 32 6.2 /
+// 7.4 / 6.7 / 9.4 / 13 / 20, at M = 512 - / - / 16.5 / 14.2 / 14.0 / 20.4, at
+// M = 2048 - / - / 47 / 41 / 39 / 38; 6912 -> 2560 at M = 64 7.9 / 10.7 /
+// 11.9 / 13.9 / 22 / 42, at M = 512 - / - / 18.7 / 15.9 / 24 / 39.
+const GemmShape kShapes4[] = {
+    {1, 2, 4, 4, 0, 0.170f, 0.170f, 1.0f, 1},  {1, 4, 8, 2, 0, 0.160f, 0.160f, 1.2f, 8},
+    {1, 5, 8, 2, 0, 0.190f, 0.190f, 1.2f, 8},  {1, 8, 8, 2, 0, 0.245f, 0.245f, 1.2f, 8},
+    {2, 8, 4, 1, 4, 0.330f, 0.270f, 0.0f, 1},  {4, 8, 4, 1, 4, 0.480f, 0.450f, 0.0f, 1},
+    {4, 16, 4, 1, 4, 0.850f, 0.830f, 0.0f, 1}, {8, 16, 4, 1, 4, 1.570f, 1.450f, 0.0f, 1},
+};
+// Pack5 (the base-3 decode is 24 vector instructions per 16 weights against
+// 9, so shapes that decode a weight once for 128 tokens pay earlier): 3200 ->
+// 8640, 32 x 128 / 64 x 128 / 128 x 128 / 128 x 256 (eight waves): M = 128
+// 15.5 / 12.2 / 16.6 / 22.1, M = 512 32 / 27.8 / 33.7 / 25.6, M = 2048 103 /
+// 77 / 83 / 75.
+const GemmShape kShapes5[] = {
+    {1, 2, 4, 4, 0, 0.290f, 0.160f, 0.0f, 1}, {1, 4, 8, 2, 0, 0.270f, 0.200f, 0.0f, 8},
+    {1, 5, 8, 2, 0, 0.310f, 0.220f, 0.0f, 8}, {1, 5, 16, 1, 0, 0.275f, 0.360f, 0.0f, 16},
+    {2, 8, 4, 1, 4, 0.650f, 0.500f, 0.0f, 1}, {4, 8, 4, 1, 4, 0.800f, 0.680f, 0.0f, 1},
+    {8, 8, 4, 1, 4, 1.300f, 1.450f, 0.0f, 1}, {8, 16, 8, 1, 4, 2.000f, 2.350f, 0.0f, 1},
+};
+
+MMConfig choose_gemm(int fmt, int M, int ngroups, int nch) {
+    // gemmw_kernel's byte offsets within a matrix and a token block are 32-bit
+    const bool wide = (size_t)ngroups * nch * kTileBytes < ((size_t)1 << 32) && nch < (1 << 16);
+    MMConfig best;
+    double best_cost = -1.0;
+    auto take = [&](const GemmShape& g) {
+        const long tiles = (long)((M + 16 * g.mb - 1) / (16 * g.mb)) * ((ngroups + g.nb - 1) / g.nb);
+        if (g.kind == 4 && (!wide || tiles > 0x7fffffff)) return;
+        const long n = (tiles + 255) / 256;  // workgroups of the busiest CU
+        const double nc = (nch + g.unit - 1) / g.unit * g.unit;
+        const double cost = g.first * nc + (double)(n - 1) * (g.rest * nc + g.gap);
+        if (best_cost >= 0.0 && cost >= best_cost) return;
+        best_cost = cost;
+        best = MMConfig{g.mb, g.nb, g.waves, g.pf, 1, g.kind};
+    };
+    if (fmt == XT_PACK5)
+        for (const GemmShape& g : kShapes5) take(g);
+    else
+        for (const GemmShape& g : kShapes4) take(g);
+    return best;
+}
+}  // namespace
+
 MMConfig choose_config(int fmt, int M, int ntiles_nb1, int nch, bool have_rowsum) {
     MMConfig c;
     if (env_config(&c)) {
@@ -2048,9 +1478,7 @@ MMConfig choose_config(int fmt, int M, int ntiles_nb1, int nch, bool have_rowsum
             c.nb = gemv_row_groups(fmt, nch, ntiles_nb1);
             return c;
         }
-        if (c.kind == 3 && M > 16 && fmt == XT_PACK4 &&
-            (nch + c.splitk - 1) / c.splitk <= gemm32_ncmax())
-            return c;
+        if (c.kind == 4 && M > 16 && gemmw_known(fmt, c.mb / 2, c.nb / (2 * c.waves), c.waves)) return c;
         if (c.kind == 0 && shape_known(c, !have_rowsum)) {
             if (c.splitk > nch) c.splitk = nch;
             return c;
@@ -2068,48 +1496,7 @@ MMConfig choose_config(int fmt, int M, int ntiles_nb1, int nch, bool have_rowsum
         }
         return MMConfig{1, 1, 8, 2, 1};
     }
-    // Prefill, Pack4 tiles: the warp-specialised 32x32x32 MFMA GEMM when K
-    // fits its LDS stage (C1 up: 10.9 -> 7.8 us).  Longer K stays on the
-    // K-split kernel below: splitting it over workgroups plus a reduction
-    // launch measured slower (C1 down: 12.6 vs 8.5 us).
-    // A grid of fewer than ~80 of its 32 x 128 tiles leaves most CUs idle
-    // while each tile takes the same ~7 us; 16 tokens x 32 rows with K over 4
-    // waves spreads such shapes over 4-8x the workgroups (M = 32: K 2560 ->
-    // N 2560 / 3840 7.2 -> 5.0 / 5.2 us; M = 24, N = 6912: 7.4 -> 6.2 us;
-    // 108 tiles, N = 13824 at M = 32: 7.8 vs 8.3 us, the GEMM stays).
-    const long g32_tiles = (long)((ntiles_nb1 * 16 + 127) / 128) * ((M + 31) / 32);
-    if (fmt == XT_PACK4 && ntiles_nb1 > 0 && g32_tiles < 80) return MMConfig{1, 2, 4, 4, 1};
-    if (fmt == XT_PACK4 && nch <= gemm32_ncmax()) {
-        c = MMConfig{2, 8, 8, 1, 1};
-        c.kind = 3;
-        return c;
-    }
-    // Prefill: the LDS GEMM when its activation slice covers K in one
-    // workgroup; otherwise 16 tokens x 64 rows per workgroup with K split
-    // over 4 waves (measured faster than split-K planes plus a reduction).
-    if (have_rowsum && nch <= gemm_ncmax(fmt)) {
-        c = MMConfig{2, 8, 4, 1, 1};
-        c.kind = 1;
-        (void)ntiles_nb1;
-        return c;
-    }
-    // Long K (activation slice too big for the GEMM's LDS): 16 tokens per
-    // workgroup, K over 8 waves, and the row-block width that fills the
-    // chip in the fewest rounds of workgroups -- e.g. C1 down (M 128, 160
-    // row groups): 80 rows -> 256 workgroups in one round, 8.6 us, against
-    // 64 rows -> 320 workgroups in two rounds, 12.5 us.
-    const int tb = (M + 15) / 16;
-    int best_nb = 4;
-    long best_cost = -1;
-    for (int nb : {4, 5, 8}) {
-        const long wgs = (long)((ntiles_nb1 + nb - 1) / nb) * tb;
-        const long cost = ((wgs + 255) / 256) * nb;
-        if (best_cost < 0 || cost < best_cost) {
-            best_cost = cost;
-            best_nb = nb;
-        }
-    }
-    return MMConfig{1, best_nb, 8, 2, 1};
+    return choose_gemm(fmt, M, ntiles_nb1, nch);
 }
 
 hipError_t launch_mm(int fmt, const MMConfig& cfg, const MMArgs& a, int ntiles_total,
