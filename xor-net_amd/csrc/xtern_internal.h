@@ -123,22 +123,20 @@ int gemv_row_groups(int fmt, int nch, int ngroups);
 bool gemv2_takes(int fmt, int nch);
 int int_gemv_waves(int fmt, int mb, int nch);
 bool gemv_fits(int fmt, int M, int nch, int waves, int ncw);
-// MLP middle stage (xtern_kernels.hip): per row of gate/up, activation,
+// MLP middle stage (xtern_mid.hip): per row of gate/up, activation,
 // optional RMSNorm, optional f32 output, optional requantisation.
 struct MidArgs {
     const float* gate;  // [M][ldg]
     const float* up;    // [M][ldg]
     int64_t ldg;
     int n;              // row length (intermediate size)
-    int C;              // set by the launcher
     int act;            // XT_ACT_*
     const float* norm_w;  // [n] RMSNorm weight, or null
     float eps;
     int mode;             // requantisation rounding (XT_QUANT_*)
-    int8_t* q;            // [M][ldq] (zero padded to ldq), or null
+    int8_t* q;            // [M][ldq] (zero padded to ldq; both multiples of 4), or null
     int ldq;
     float* inv;           // [M]
-    int32_t* rowsum;      // [M] or null
     float* out;           // [M][ldo] f32 activation (+ norm) result, or null
     int64_t ldo;
 };

@@ -1603,620 +1603,3 @@ hipError_t launch_hf_tiles(int fmt, const uint8_t* stored, int64_t K, int64_t N,
 }
 
 }  // namespace xt
-
-
-namespace xt {
-
-// ---------------------------------------------------------------------------
-// MLP middle: activation, optional RMSNorm, requantisation
-// ---------------------------------------------------------------------------
-
-// expf of the C library the reference links (glibc 2.28+, from ARM's
-// optimized-routines): x * 32/ln2 rounded to an integer k, 2^(k/32) from a
-// 32-entry table with k/32's integer part added to the exponent bits, and a
-// cubic in the remainder, all in double, rounded once to float.  The two
-// products with InvLn2N are fused multiply-adds, as the FMA build of the
-// library compiles them.  Equal to the host expf on every one of the 2^32
-// float inputs (checked exhaustively on the build host).
-__constant__ uint64_t kExp2Tab[32] = {
-    0x3ff0000000000000ULL, 0x3fefd9b0d3158574ULL, 0x3fefb5586cf9890fULL, 0x3fef9301d0125b51ULL,
-    0x3fef72b83c7d517bULL, 0x3fef54873168b9aaULL, 0x3fef387a6e756238ULL, 0x3fef1e9df51fdee1ULL,
-    0x3fef06fe0a31b715ULL, 0x3feef1a7373aa9cbULL, 0x3feedea64c123422ULL, 0x3feece086061892dULL,
-    0x3feebfdad5362a27ULL, 0x3feeb42b569d4f82ULL, 0x3feeab07dd485429ULL, 0x3feea47eb03a5585ULL,
-    0x3feea09e667f3bcdULL, 0x3fee9f75e8ec5f74ULL, 0x3feea11473eb0187ULL, 0x3feea589994cce13ULL,
-    0x3feeace5422aa0dbULL, 0x3feeb737b0cdc5e5ULL, 0x3feec49182a3f090ULL, 0x3feed503b23e255dULL,
-    0x3feee89f995ad3adULL, 0x3feeff76f2fb5e47ULL, 0x3fef199bdd85529cULL, 0x3fef3720dcef9069ULL,
-    0x3fef5818dcfba487ULL, 0x3fef7c97337b9b5fULL, 0x3fefa4afa2a490daULL, 0x3fefd0765b6e4540ULL};
-
-__device__ __forceinline__ float libc_expf(float x) {
-    const uint32_t ux = __float_as_uint(x);
-    const uint32_t top = (ux >> 20) & 0x7ffu;
-    if (top >= 0x42bu) {  // |x| >= 88, inf, NaN
-        if (ux == 0xff800000u) return 0.0f;
-        if (top >= 0x7f8u) return x + x;
-        if (x > 0x1.62e42ep6f) return __builtin_inff();
-        if (x < -0x1.9fe368p6f) return 0.0f;
-    }
-    const double C0 = 0x1.c6af84b912394p-5 / 32 / 32 / 32, C1 = 0x1.ebfce50fac4f3p-3 / 32 / 32,
-                 C2 = 0x1.62e42ff0c52d6p-1 / 32;
-    const double inv = 0x1.71547652b82fep+0 * 32, shift = 0x1.8p+52;
-    const double xd = (double)x;
-    double kd = __fma_rn(inv, xd, shift);
-    const uint64_t ki = (uint64_t)__double_as_longlong(kd);
-    kd = __dsub_rn(kd, shift);
-    const double r = __fma_rn(inv, xd, -kd);
-    const uint64_t t = kExp2Tab[ki & 31] + (ki << 47);
-    const double s = __longlong_as_double((long long)t);
-    const double z = __fma_rn(C0, r, C1);
-    const double r2 = __dmul_rn(r, r);
-    double y = __fma_rn(C2, r, 1.0);
-    y = __fma_rn(z, r2, y);
-    return (float)__dmul_rn(y, s);
-}
-
-// quantization.rs:213 / :280: g * (1 / (1 + exp(-g))) * u.
-__device__ __forceinline__ float silu_scalar(float g, float u) {
-    const float sig = __fdiv_rn(1.0f, __fadd_rn(1.0f, libc_expf(-g)));
-    return __fmul_rn(__fmul_rn(g, sig), u);
-}
-// tensor.rs:186-188: (x / (1 + exp(-x))) * u.
-__device__ __forceinline__ float silu_div(float g, float u) {
-    return __fmul_rn(__fdiv_rn(g, __fadd_rn(1.0f, libc_expf(-g))), u);
-}
-// quantization.rs:215-216, :268-270; tensor.rs:223-224: max(g, 0)^2 * u.
-__device__ __forceinline__ float relu2_mul(float g, float u) {
-    const float r = (g > 0.0f) ? g : 0.0f;
-    return __fmul_rn(__fmul_rn(r, r), u);
-}
-// One lane of silu_inplace_avx512's vector body (quantization.rs:243-272).
-__device__ __forceinline__ float silu_poly(float g, float u) {
-    const float inv_ln2 = 1.44269504088896341f, ln2 = 0.693147180559945309f;
-    const float hi = 88.3762626647949f, lo = -88.3762626647949f;
-    float x = __fsub_rn(0.0f, g);
-    x = (x < hi) ? x : hi;  // MINPS: second operand unless x < hi (NaN -> hi)
-    x = (x > lo) ? x : lo;  // MAXPS
-    const float fx = __fmul_rn(x, inv_ln2);
-    const float n_f = __builtin_rintf(fx);
-    const float t = __fsub_rn(x, __fmul_rn(n_f, ln2));
-    float e = __fmaf_rn(1.0f / 24.0f, t, 1.0f / 6.0f);
-    e = __fmaf_rn(e, t, 0.5f);
-    e = __fmaf_rn(e, t, 1.0f);
-    e = __fmaf_rn(e, t, 1.0f);
-    const uint32_t bits = ((uint32_t)(int)n_f + 127u) << 23;
-    const float exp_x = __fmul_rn(e, __uint_as_float(bits));
-    const float sig = __fdiv_rn(1.0f, __fadd_rn(1.0f, exp_x));
-    return __fmul_rn(__fmul_rn(g, sig), u);
-}
-
-__device__ __forceinline__ float apply_act(int act, float g, float u, bool main_lane) {
-    switch (act) {
-        case XT_ACT_SILU_INPLACE_AVX512:
-            return main_lane ? silu_poly(g, u) : silu_scalar(g, u);
-        case XT_ACT_SILU_INPLACE_SCALAR:
-            return silu_scalar(g, u);
-        case XT_ACT_SILU_MUL:
-            return silu_div(g, u);
-        case kActIdentity:
-            return g;
-        default:
-            return relu2_mul(g, u);
-    }
-}
-
-constexpr int kMidThreads = 1024;
-constexpr int kMidWaves = kMidThreads / 64;
-constexpr int kMidCmax = 16;                         // row length <= 16 * 1024
-constexpr int kMidRecMax = 1024;                     // piece records in LDS
-constexpr uint32_t kGrid = 1u << 24;                 // grid points per binade
-
-// Wave-wide data movement with DPP (gfx9 encodings): row_shr:n = 0x110 + n
-// shifts within rows of 16 lanes, row_bcast:15 / row_bcast:31 = 0x142 / 0x143
-// broadcast lane 15 / 31 into the following rows, wave_shr:1 = 0x138 and
-// wave_shl:1 = 0x130 shift across the whole wave.  Lanes without a source
-// (or outside ROW_MASK) receive 0.
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ uint32_t dpp32(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROW_MASK, 0xf, false);
-}
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ uint64_t dpp64(uint64_t v) {
-    const uint32_t lo = dpp32<CTRL, ROW_MASK>((uint32_t)v);
-    const uint32_t hi = dpp32<CTRL, ROW_MASK>((uint32_t)(v >> 32));
-    return ((uint64_t)hi << 32) | lo;
-}
-
-// Inclusive wave scans (Hillis-Steele in rows of 16, then row broadcasts).
-__device__ __forceinline__ uint64_t wave_scan_add(uint64_t v) {
-    v += dpp64<0x111, 0xf>(v);
-    v += dpp64<0x112, 0xf>(v);
-    v += dpp64<0x114, 0xf>(v);
-    v += dpp64<0x118, 0xf>(v);
-    v += dpp64<0x142, 0xa>(v);
-    v += dpp64<0x143, 0xc>(v);
-    return v;
-}
-__device__ __forceinline__ uint32_t wave_scan_add(uint32_t v) {
-    v += dpp32<0x111, 0xf>(v);
-    v += dpp32<0x112, 0xf>(v);
-    v += dpp32<0x114, 0xf>(v);
-    v += dpp32<0x118, 0xf>(v);
-    v += dpp32<0x142, 0xa>(v);
-    v += dpp32<0x143, 0xc>(v);
-    return v;
-}
-// Wave maximum of non-negative floats (0 is the identity), in every lane.
-__device__ __forceinline__ float wave_max_nonneg(float v) {
-    v = fmaxf(v, __uint_as_float(dpp32<0x111, 0xf>(__float_as_uint(v))));
-    v = fmaxf(v, __uint_as_float(dpp32<0x112, 0xf>(__float_as_uint(v))));
-    v = fmaxf(v, __uint_as_float(dpp32<0x114, 0xf>(__float_as_uint(v))));
-    v = fmaxf(v, __uint_as_float(dpp32<0x118, 0xf>(__float_as_uint(v))));
-    v = fmaxf(v, __uint_as_float(dpp32<0x142, 0xa>(__float_as_uint(v))));
-    v = fmaxf(v, __uint_as_float(dpp32<0x143, 0xc>(__float_as_uint(v))));
-    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), 63));
-}
-__device__ __forceinline__ int wave_sum_int(int v) {
-    const uint32_t s = wave_scan_add((uint32_t)v);
-    return (int)__builtin_amdgcn_readlane(s, 63);
-}
-template <typename T>
-__device__ __forceinline__ T lane_read(T v, int k) {
-    if constexpr (sizeof(T) == 8) {
-        const uint64_t b = __builtin_bit_cast(uint64_t, v);
-        const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)b, k);
-        const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(b >> 32), k);
-        return __builtin_bit_cast(T, ((uint64_t)hi << 32) | lo);
-    } else {
-        return __builtin_bit_cast(T, __builtin_amdgcn_readlane(__builtin_bit_cast(uint32_t, v), k));
-    }
-}
-
-// Integer increment of adding t (finite, >= 0) to a running sum on the grid
-// u = 2^(b-23): q = floor(t / u) (capped at 2^24), r = 0 below half, 1 at an
-// exact half, 2 above.
-__device__ __forceinline__ void grid_split(float t, int b, uint32_t* q, int* r) {
-    const uint32_t bits = __float_as_uint(t);
-    const uint32_t ef = (bits >> 23) & 0xffu;
-    const uint32_t m = ef ? ((bits & 0x7fffffu) | 0x800000u) : (bits & 0x7fffffu);
-    const int et = ef ? (int)ef - 150 : -149;
-    const int shift = (b - 23) - et;
-    // shift <= 0: t is a multiple of u (q = m << -shift, capped at 2^24)
-    const int ls = min(-shift, 24);
-    const uint32_t qup = min(m << max(ls, 0), kGrid);
-    // shift > 0: m < 2^24, so shifts of 25 or more leave q = 0, remainder m
-    const int sc = min(max(shift, 1), 25);
-    const uint32_t qdn = m >> sc;
-    const uint32_t rem = m & ((1u << sc) - 1u), half = 1u << (sc - 1);
-    const int rdn = rem < half ? 0 : (rem == half ? 1 : 2);
-    *q = shift <= 0 ? (m ? qup : 0u) : qdn;
-    *r = shift <= 0 ? 0 : rdn;
-}
-
-struct SeqSumLds {
-    float wtot[kMidWaves];
-    uint64_t wgp[kMidWaves];
-    int wcnt[kMidWaves];
-    float res;
-};
-
-__device__ __forceinline__ float wave_scan_addf(float v) {
-    v = __fadd_rn(v, __uint_as_float(dpp32<0x111, 0xf>(__float_as_uint(v))));
-    v = __fadd_rn(v, __uint_as_float(dpp32<0x112, 0xf>(__float_as_uint(v))));
-    v = __fadd_rn(v, __uint_as_float(dpp32<0x114, 0xf>(__float_as_uint(v))));
-    v = __fadd_rn(v, __uint_as_float(dpp32<0x118, 0xf>(__float_as_uint(v))));
-    v = __fadd_rn(v, __uint_as_float(dpp32<0x142, 0xa>(__float_as_uint(v))));
-    v = __fadd_rn(v, __uint_as_float(dpp32<0x143, 0xc>(__float_as_uint(v))));
-    return v;
-}
-// Binade of a float >= 0 (subnormals and 0 in -126, infinity 128).
-__device__ __forceinline__ int binade_f(float a) {
-    const int e = (int)(__float_as_uint(a) >> 23);
-    return e == 0 ? -126 : e - 127;
-}
-
-// Significand of s >= 0 on the grid of its binade (implicit bit included;
-// for binade -126 the subnormal or smallest-normal encoding), and the float
-// of significand T < 2^24 in binade b.
-__device__ __forceinline__ int sig_binade(float s, uint32_t* S) {
-    const uint32_t sbits = __float_as_uint(s);
-    const int se = (int)(sbits >> 23);
-    *S = (sbits & 0x7fffffu) | (se ? 0x800000u : 0u);
-    return se == 0 ? -126 : se - 127;
-}
-__device__ __forceinline__ float from_grid(uint64_t T, int b) {
-    return __uint_as_float(T >= 0x800000u ? ((uint32_t)(b + 127) << 23) | ((uint32_t)T & 0x7fffffu)
-                                          : (uint32_t)T);  // b = -126, subnormal
-}
-
-// s + lt[j] + ... + lt[end - 1], each partial sum rounded to f32, by one
-// whole wave (s is the same in every lane): 256 elements at a time (4
-// consecutive ones per lane) are split on the grid of the running sum's
-// binade and prefix-summed; the leading ones that are no tie and keep the sum
-// inside the binade are added at once (exact integer addition on the grid),
-// the next one with a real f32 add.
-__device__ float seq_advance(float s, const float* lt, int j, int end) {
-    const int lane = threadIdx.x & 63;
-    s = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(s)));
-    while (j < end) {
-        uint32_t S;
-        const int bs = sig_binade(s, &S);
-        if (bs > 127) return s;  // infinity plus finite non-negative terms
-        // lane l: elements j + 4 l .. j + 4 l + 3; local inclusive prefixes
-        uint32_t pre[4];
-        int kbad = 4;  // first element of the lane that is a tie or past `end`
-        uint32_t acc = 0;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int e = j + 4 * lane + k;
-            uint32_t q = 0;
-            int r = 1;  // past the end: treated as a stop
-            if (e < end) grid_split(lt[e], bs, &q, &r);
-            if (r == 1 && kbad == 4) kbad = k;
-            acc += min(q + (r == 2 ? 1u : 0u), kGrid);
-            pre[k] = acc;  // <= 4 * 2^24 per lane
-        }
-        const uint32_t lincl = wave_scan_add(acc);  // <= 256 * 2^24 < 2^32
-        const uint32_t lexcl = lincl - acc;
-        // first element (in order) that is a stop or leaves the binade
-        int kfirst = kbad;
-#pragma unroll
-        for (int k = 3; k >= 0; --k)
-            if ((uint64_t)S + lexcl + pre[k] >= kGrid) kfirst = min(kfirst, k);
-        const uint64_t bad = __ballot(kfirst < 4);
-        int m;  // elements added on the grid
-        uint32_t pm = 0;
-        if (bad) {
-            const int L = (int)__builtin_ctzll(bad);
-            const int kL = lane_read(kfirst, L);
-            m = 4 * L + kL;
-            if (m > 0) {
-                // prefix through element m - 1
-                uint32_t mine = 0;
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (k == kL - 1) mine = lexcl + pre[k];
-                pm = kL > 0 ? lane_read(mine, L) : lane_read(lincl, L - 1);
-            }
-        } else {
-            m = 256;
-            pm = lane_read(lincl, 63);
-        }
-        if (m > 0) {
-            s = from_grid((uint64_t)S + pm, bs);
-            j += m;
-        }
-        if (m < 256 && j < end) {
-            s = __fadd_rn(s, lt[j]);
-            ++j;
-        }
-        s = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(s)));
-    }
-    return s;
-}
-
-// Sequential float sum t[0] + t[1] + ... + t[n-1] (each partial sum rounded
-// to f32, in index order) -- the order of rms_norm's sum of squares --
-// computed by the whole workgroup.  Within one binade [2^b, 2^(b+1)) of the
-// running sum, every f32 add is an integer add on the grid u = 2^(b-23):
-// fl(s + t) = s + u * round(t / u), except when t / u is an exact half (a
-// tie, whose rounding depends on the parity of s) or when the sum leaves the
-// binade.  So:
-//  1. a float prefix sum predicts the binade of the running sum before each
-//     element;
-//  2. elements that are ties, or after which the predicted binade changes,
-//     end a "piece"; every other element contributes its integer increment,
-//     and the increments are prefix-summed;
-//  3. one wave walks the pieces in order with the running sum's bits on the
-//     scalar unit: if they lie in the piece's precomputed range (the sum is
-//     in the predicted binade and stays below its top after the piece), the
-//     piece is one integer add on the bits; otherwise seq_advance adds the
-//     piece; the piece's end element is always a real f32 add.
-// The result never depends on the prediction being right, only the speed
-// does.  `lt` holds t[0..n) (finite, >= 0) in LDS; thread j handles the
-// contiguous elements [j*E, j*E + E), E = ceil(n / 1024) <= CM.
-template <int CM>
-__device__ __forceinline__ float exact_seq_sum(int n, const float* lt, SeqSumLds& sl, int* rec_idx,
-                                               uint64_t* rec_gp, int* rec_b) {
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int E = (n + kMidThreads - 1) / kMidThreads;
-    const int i0 = tid * E;
-    const int cnt = max(0, min(E, n - i0));  // this thread's elements: [i0, i0 + cnt)
-    float t[CM];
-#pragma unroll
-    for (int e = 0; e < CM; ++e) t[e] = e < cnt ? lt[i0 + e] : 0.0f;
-    // 1. prefix sums: thread-local, then across lanes and waves
-    float acc = 0.0f;
-#pragma unroll
-    for (int e = 0; e < CM; ++e)
-        if (e < cnt) acc = __fadd_rn(acc, t[e]);
-    const float incl = wave_scan_addf(acc);
-    const float excl = __uint_as_float(dpp32<0x138, 0xf>(__float_as_uint(incl)));  // wave_shr:1
-    const float excl_next = __uint_as_float(dpp32<0x130, 0xf>(__float_as_uint(excl)));  // wave_shl:1
-    if (lane == 63) sl.wtot[w] = incl;
-    __syncthreads();
-    float woff = 0.0f;
-    for (int j = 0; j < w; ++j) woff = __fadd_rn(woff, sl.wtot[j]);
-    const float woff_next = __fadd_rn(woff, sl.wtot[w]);
-    // Prefix before this thread's first element, and before the next
-    // thread's first element, computed exactly as that thread computes it.
-    const float off = __fadd_rn(woff, excl);
-    const float off_next = lane < 63 ? __fadd_rn(woff, excl_next) : __fadd_rn(woff_next, 0.0f);
-
-    // 2. The binade before element i is that of off + (local prefix before
-    // i) -- the next thread's `off` after the last element.  Piece ends and
-    // integer increments, kept in registers.
-    uint32_t inc[CM];
-    int bb[CM];
-    uint32_t endbits = 0;
-    uint64_t dsum = 0;
-    {
-        float lp = 0.0f;
-        int b = binade_f(off);
-#pragma unroll
-        for (int e = 0; e < CM; ++e) {
-            inc[e] = 0;
-            bb[e] = b;
-            if (e < cnt) {
-                lp = __fadd_rn(lp, t[e]);
-                const int bn = (e + 1 < E) ? binade_f(__fadd_rn(off, lp)) : binade_f(off_next);
-                uint32_t q;
-                int r;
-                grid_split(t[e], b, &q, &r);
-                const bool end = r == 1 || bn != b || i0 + e == n - 1;
-                inc[e] = end ? 0u : min(q + (r == 2 ? 1u : 0u), kGrid);
-                endbits |= (end ? 1u : 0u) << e;
-                dsum += inc[e];
-                b = bn;
-            }
-        }
-    }
-    const uint32_t ends = __builtin_popcount(endbits);
-    const uint64_t gincl = wave_scan_add(dsum);
-    const uint32_t cincl = wave_scan_add(ends);
-    if (lane == 63) {
-        sl.wgp[w] = gincl;
-        sl.wcnt[w] = (int)cincl;
-    }
-    __syncthreads();
-    uint64_t gp = gincl - dsum;
-    int rank = (int)(cincl - ends);
-    int total_ends = 0;
-    for (int j = 0; j < kMidWaves; ++j) {
-        if (j < w) {
-            gp += sl.wgp[j];
-            rank += sl.wcnt[j];
-        }
-        total_ends += sl.wcnt[j];
-    }
-    const bool overflow = total_ends > kMidRecMax;
-    if (!overflow && endbits) {
-#pragma unroll
-        for (int e = 0; e < CM; ++e) {
-            if (e < cnt) {
-                if ((endbits >> e) & 1u) {
-                    rec_idx[rank] = i0 + e;
-                    rec_gp[rank] = gp;  // own increment is 0
-                    rec_b[rank] = bb[e];
-                    ++rank;
-                }
-                gp += inc[e];
-            }
-        }
-    }
-    __syncthreads();
-
-    // 3. walk the pieces (wave 0).  Records are loaded 64 at a time, one per
-    // lane, with everything that does not depend on the running sum: the
-    // range [lo, lim) of running-sum bits for which the piece's P increments
-    // are one integer add on the bits (in binade b the bits are
-    // ((b + 127) << 23) + significand - 2^23, or the significand itself for
-    // b = -126, so "sum in binade b and sum + P below 2^(b+1)" is
-    // lo <= bits < hi - P).  The sequential part reads them with readlane.
-    if (w == 0) {
-        // (uniform values read from LDS are made scalar, so that the walk
-        // runs on the scalar unit instead of under exec masks)
-        total_ends = __builtin_amdgcn_readfirstlane(total_ends);
-        float s = 0.0f;
-        if (overflow) {
-            s = seq_advance(0.0f, lt, 0, n);
-        } else {
-            uint32_t sbits = 0;
-            for (int k0 = 0; k0 < total_ends; k0 += 64) {
-                const int k = k0 + lane;
-                int idx = 0, start = 0;
-                uint32_t lo = 0, lim = 0xffffffffu, P32 = 0;
-                float tend = 0.0f;
-                if (k < total_ends) {
-                    idx = rec_idx[k];
-                    const int rb = rec_b[k];
-                    start = k > 0 ? rec_idx[k - 1] + 1 : 0;
-                    const uint64_t P = rec_gp[k] - (k > 0 ? rec_gp[k - 1] : 0ull);
-                    tend = lt[idx];
-                    if (start < idx) {
-                        const uint32_t hi = (uint32_t)(rb + 128) << 23;
-                        lo = rb == -126 ? 0u : (uint32_t)(rb + 127) << 23;
-                        if (rb > 127 || P >= (uint64_t)(hi - lo)) {
-                            lo = 1u;  // empty range
-                            lim = 0u;
-                        } else {
-                            lim = hi - (uint32_t)P;
-                            P32 = (uint32_t)P;
-                        }
-                    }
-                }
-                const int kn = min(64, total_ends - k0);
-                // The dependency chain per piece is two compares, a select
-                // and one f32 add; the fallback is a branch not taken.
-                for (int kk = 0; kk < kn; ++kk) {
-                    const uint32_t klo = lane_read(lo, kk), klim = lane_read(lim, kk);
-                    const uint32_t kp = lane_read(P32, kk);
-                    const float kt = lane_read(tend, kk);
-                    const bool inr = sbits >= klo && sbits < klim;
-                    sbits = inr ? sbits + kp : sbits;
-                    if (__builtin_expect(!inr, 0)) {
-                        sbits = __float_as_uint(seq_advance(__uint_as_float(sbits), lt,
-                                                            lane_read(start, kk), lane_read(idx, kk)));
-                    }
-                    sbits = __float_as_uint(__fadd_rn(__uint_as_float(sbits), kt));
-                }
-            }
-            s = __uint_as_float(sbits);
-        }
-        if (lane == 0) sl.res = s;
-    }
-    __syncthreads();
-    return sl.res;
-}
-
-// One workgroup (16 waves) per row.  Element i = (wave*C + c)*64 + lane is
-// held in registers from the load to the quantisation.
-template <int ACT, int CM>
-__global__ __launch_bounds__(kMidThreads) void mlp_mid_kernel(MidArgs a) {
-    extern __shared__ __align__(16) uint8_t lds[];
-    __shared__ SeqSumLds sl;
-    __shared__ float sm_f[kMidWaves];
-    __shared__ int sm_i[kMidWaves];
-    const int m = blockIdx.x;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int n = a.n, C = a.C;
-    const int nmain = (n / 16) * 16;
-    const float* gr = a.gate + (size_t)m * a.ldg;
-    const float* ur = a.up + (size_t)m * a.ldg;
-    float v[CM], nwv[CM];
-#pragma unroll
-    for (int c = 0; c < CM; ++c) {
-        const int i = (w * C + c) * 64 + lane;
-        v[c] = (c < C && i < n) ? apply_act(ACT, gr[i], ACT == kActIdentity ? 0.0f : ur[i], i < nmain)
-                                : 0.0f;
-        nwv[c] = (a.norm_w && c < C && i < n) ? a.norm_w[i] : 0.0f;  // fetched early
-    }
-    if (a.norm_w) {
-        float* lt = reinterpret_cast<float*>(lds);
-        int* rec_idx = reinterpret_cast<int*>(lds + (size_t)C * kMidThreads * 4);
-        int* rec_b = rec_idx + kMidRecMax;
-        uint64_t* rec_gp = reinterpret_cast<uint64_t*>(rec_b + kMidRecMax);
-        bool bad_nan = false, bad_inf = false;
-#pragma unroll
-        for (int c = 0; c < CM; ++c) {
-            const int i = (w * C + c) * 64 + lane;
-            const float t = __fmul_rn(v[c], v[c]);
-            if (c < C && i < n) {
-                lt[i] = t;
-                bad_nan |= (t != t);
-                bad_inf |= (bool)__builtin_isinf(t);
-            }
-        }
-        const int wf = (__ballot(bad_nan) ? 1 : 0) | (__ballot(bad_inf) ? 2 : 0);
-        if (lane == 0) sm_i[w] = wf;
-        __syncthreads();
-        int flags = 0;
-#pragma unroll
-        for (int j = 0; j < kMidWaves; ++j) flags |= sm_i[j];
-        float sum;
-        if (flags & 1) sum = __builtin_nanf("");
-        else if (flags & 2) sum = __builtin_inff();
-        else sum = exact_seq_sum<CM>(n, lt, sl, rec_idx, rec_gp, rec_b);
-        // fast_attention_simd.rs:485-486.  sqrtf is correctly rounded on the
-        // host; the hardware f32 square root is not, so take the correctly
-        // rounded double root and round it once (exact: 53 >= 2*24 + 2).
-        const float ms = __fadd_rn(__fdiv_rn(sum, (float)n), a.eps);
-        const float rms = (float)__dsqrt_rn((double)ms);
-        const float invr = __fdiv_rn(1.0f, rms);
-#pragma unroll
-        for (int c = 0; c < CM; ++c) {
-            const int i = (w * C + c) * 64 + lane;
-            if (c < C && i < n) v[c] = __fmul_rn(__fmul_rn(v[c], invr), nwv[c]);
-        }
-    }
-    if (a.out) {
-        float* orow = a.out + (size_t)m * a.ldo;
-#pragma unroll
-        for (int c = 0; c < CM; ++c) {
-            const int i = (w * C + c) * 64 + lane;
-            if (c < C && i < n) orow[i] = v[c];
-        }
-    }
-    if (!a.q) return;
-    float mx = 0.0f;
-#pragma unroll
-    for (int c = 0; c < CM; ++c) mx = fmaxf(mx, fabsf(v[c]));
-    mx = wave_max_nonneg(mx);
-    if (lane == 0) sm_f[w] = mx;
-    __syncthreads();
-    mx = 0.0f;
-#pragma unroll
-    for (int j = 0; j < kMidWaves; ++j) mx = fmaxf(mx, sm_f[j]);
-    const float scale = (mx > 0.0f) ? __fdiv_rn(127.0f, mx) : 1.0f;
-    const float invs = (mx > 0.0f) ? __fdiv_rn(mx, 127.0f) : 1.0f;
-    int8_t* qr = a.q + (size_t)m * a.ldq;
-    int sum = 0;
-    // (the rounding mode is chosen once, so that only one quantiser's code
-    // runs through the unrolled loop)
-    auto quant_row = [&](auto mode_c) {
-#pragma unroll
-        for (int c = 0; c < CM; ++c) {
-            const int i = (w * C + c) * 64 + lane;
-            if (c < C && i < n) {
-                const int b = quant_one(v[c], scale, decltype(mode_c)::value, i < nmain);
-                qr[i] = (int8_t)b;
-                sum += b;
-            }
-        }
-    };
-    if (a.mode == XT_QUANT_AVX512) quant_row(std::integral_constant<int, XT_QUANT_AVX512>{});
-    else quant_row(std::integral_constant<int, XT_QUANT_SCALAR>{});
-    for (int i = n + tid; i < a.ldq; i += kMidThreads) qr[i] = 0;
-    if (!a.rowsum) {  // the product decodes signed weights or sums the row itself
-        if (tid == 0) a.inv[m] = invs;
-        return;
-    }
-    sum = wave_sum_int(sum);
-    __syncthreads();  // sm_i reuse after the flag reads
-    if (lane == 0) sm_i[w] = sum;
-    __syncthreads();
-    if (tid == 0) {
-        int tot = 0;
-        for (int j = 0; j < kMidWaves; ++j) tot += sm_i[j];
-        a.inv[m] = invs;
-        if (a.rowsum) a.rowsum[m] = tot;
-    }
-}
-
-int mid_max_cols() { return kMidCmax * kMidThreads; }
-
-hipError_t launch_mlp_mid(const MidArgs& a0, int M, hipStream_t s) {
-    if (M <= 0) return hipSuccess;
-    MidArgs a = a0;
-    a.C = (a.n + kMidThreads - 1) / kMidThreads;
-    if (a.n <= 0 || a.C > kMidCmax) return hipErrorInvalidValue;
-    const size_t lds = a.norm_w ? (size_t)a.C * kMidThreads * 4 + (size_t)kMidRecMax * 16 : 0;
-    // Elements per thread, rounded up to a compiled bound: every per-element
-    // loop is unrolled to the bound and runs once, so the smallest bound
-    // means the least straight-line code to fetch (measured: n = 6912 with
-    // bound 8 instead of 16, 2.8 us less per row).
-    const int cm = a.C <= 2 ? 2 : a.C <= 4 ? 4 : a.C <= 8 ? 8 : 16;
-#define XT_MID(ACT_, CM_) \
-    hipLaunchKernelGGL((mlp_mid_kernel<ACT_, CM_>), dim3(M), dim3(kMidThreads), lds, s, a)
-#define XT_MID_CM(ACT_)                 \
-    switch (cm) {                       \
-        case 2: XT_MID(ACT_, 2); break; \
-        case 4: XT_MID(ACT_, 4); break; \
-        case 8: XT_MID(ACT_, 8); break; \
-        default: XT_MID(ACT_, 16); break; \
-    }
-    switch (a.act) {
-        case XT_ACT_RELU2_MUL: XT_MID_CM(XT_ACT_RELU2_MUL) break;
-        case XT_ACT_SILU_INPLACE_AVX512: XT_MID_CM(XT_ACT_SILU_INPLACE_AVX512) break;
-        case XT_ACT_SILU_INPLACE_SCALAR: XT_MID_CM(XT_ACT_SILU_INPLACE_SCALAR) break;
-        case XT_ACT_SILU_MUL: XT_MID_CM(XT_ACT_SILU_MUL) break;
-        case kActIdentity: XT_MID_CM(kActIdentity) break;
-        default:
-            return hipErrorInvalidValue;
-    }
-#undef XT_MID_CM
-#undef XT_MID
-    return hipGetLastError();
-}
-
-}  // namespace xt
-
-
