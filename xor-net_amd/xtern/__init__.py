@@ -266,26 +266,44 @@ def encode_sparse_row(vals, in_dim):
 # Device weights and raw entry points
 # ---------------------------------------------------------------------------
 
+# A call's host path is a large part of a small call's time (one projection of
+# one token: 3.9 us on the GPU): plain integers where ctypes takes a pointer,
+# the current stream's handle without a Stream object (0.2 against 2.8 us), no
+# views of tensors that are [rows, columns] already.  12.0 -> 6.5 us a call.
+
 def _torch():
-    import torch
-    return torch
+    if _torch_mod is None:
+        raise ImportError("torch is needed for device tensors")
+    return _torch_mod
+
+
+try:
+    _raw_stream, _cur_device = _torch_mod._C._cuda_getCurrentRawStream, _torch_mod._C._cuda_getDevice
+except AttributeError:  # (a torch without them, or none)
+    _raw_stream = None
 
 
 def _stream_ptr(stream=None):
-    torch = _torch()
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    if stream is not None:
+        return stream.cuda_stream
+    if _raw_stream is None:
+        return _torch().cuda.current_stream().cuda_stream
+    return _raw_stream(_cur_device())
 
 
 def _dev_ptr(t, dtype, what):
-    torch = _torch()
-    if not isinstance(t, torch.Tensor) or not t.is_cuda:
+    if not isinstance(t, _torch().Tensor) or not t.is_cuda:
         raise XternError(XT_ERR_INVALID, f"{what} must be a CUDA (HIP) tensor")
     if t.dtype != dtype:
         raise XternError(XT_ERR_INVALID, f"{what} must be {dtype}, got {t.dtype}")
     if not t.is_contiguous():
         raise XternError(XT_ERR_INVALID, f"{what} must be contiguous")
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
+
+
+def _rows(x):
+    """x as [rows, columns]."""
+    return x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
 
 
 class DeviceWeights:
@@ -545,7 +563,7 @@ def quantize_i8(x, mode=XT_QUANT_AVX512, stream=None):
     """Device quantize_f32_to_i8 over the rows of x [M, K] (or [K]).
     Returns (q int8 [M, K], inv_scale f32 [M])."""
     torch = _torch()
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = _rows(x)
     M, K = x2.shape
     q = torch.empty((M, K), dtype=torch.int8, device=x.device)
     inv = torch.empty((M,), dtype=torch.float32, device=x.device)
@@ -558,7 +576,7 @@ def quantize_i8(x, mode=XT_QUANT_AVX512, stream=None):
 def quantize_i8_rowsum(x, mode=XT_QUANT_AVX512, stream=None):
     """quantize_i8 plus the exact i32 row sums of q (an xtern extension)."""
     torch = _torch()
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = _rows(x)
     M, K = x2.shape
     q = torch.empty((M, K), dtype=torch.int8, device=x.device)
     inv = torch.empty((M,), dtype=torch.float32, device=x.device)
@@ -574,7 +592,7 @@ def quantize_i8_rowsum(x, mode=XT_QUANT_AVX512, stream=None):
 def linear_q_rowsum(w, q, inv, rowsum, out=None, stream=None):
     """linear_q with caller-provided row sums of q (an xtern extension)."""
     torch = _torch()
-    q2 = q.reshape(-1, q.shape[-1])
+    q2 = _rows(q)
     M = q2.shape[0]
     y = out if out is not None else torch.empty((M, w.out_dim), dtype=torch.float32, device=q.device)
     _check(_lib.xt_ternary_linear_q_rowsum(w.handle, _dev_ptr(q2, torch.int8, "q"),
@@ -588,7 +606,7 @@ def linear_q_rowsum(w, q, inv, rowsum, out=None, stream=None):
 def linear_q(w, q, inv, acc=False, out=None, stream=None):
     """y = dot(q, W) * inv * w_scales for q [M, K] int8, inv [M] f32."""
     torch = _torch()
-    q2 = q.reshape(-1, q.shape[-1])
+    q2 = _rows(q)
     M = q2.shape[0]
     if q2.shape[1] != w.in_dim:
         raise XternError(XT_ERR_INVALID,
@@ -607,7 +625,7 @@ def linear_f32_noalloc(w, x, mode=XT_QUANT_AVX512, out=None, stream=None):
     """linear_f32 through xt_ternary_linear_f32_noalloc (static device scratch,
     no allocation in the library; calls overlapping on one GPU race)."""
     torch = _torch()
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = _rows(x)
     M = x2.shape[0]
     y = out if out is not None else torch.empty((M, w.out_dim), dtype=torch.float32, device=x.device)
     _check(_lib.xt_ternary_linear_f32_noalloc(w.handle, _dev_ptr(x2, torch.float32, "x"), M,
@@ -624,14 +642,15 @@ def workspace_release():
 def linear_f32(w, x, mode=XT_QUANT_AVX512, out=None, stream=None):
     """Quantise rows of x [M, K] f32 and apply the ternary product."""
     torch = _torch()
-    x2 = x.reshape(-1, x.shape[-1])
-    M = x2.shape[0]
-    if x2.shape[1] != w.in_dim:
+    f32 = torch.float32
+    x2 = _rows(x)
+    M, K = x2.shape
+    if K != w.in_dim:
         raise XternError(XT_ERR_INVALID,
-                         f"Input dimension mismatch: expected {w.in_dim}, got {x2.shape[1]}")
-    y = out if out is not None else torch.empty((M, w.out_dim), dtype=torch.float32, device=x.device)
-    _check(_lib.xt_ternary_linear_f32(w.handle, _dev_ptr(x2, torch.float32, "x"), M,
-                                      _dev_ptr(y, torch.float32, "y"), mode, _stream_ptr(stream)))
+                         f"Input dimension mismatch: expected {w.in_dim}, got {K}")
+    y = out if out is not None else torch.empty((M, w.out_dim), dtype=f32, device=x.device)
+    _check(_lib.xt_ternary_linear_f32(w.handle, _dev_ptr(x2, f32, "x"), M, _dev_ptr(y, f32, "y"),
+                                      mode, _stream_ptr(stream)))
     return y
 
 
@@ -656,7 +675,7 @@ def rms_norm(x, weight, eps, out=None, stream=None):
     if weight.numel() != n:
         raise XternError(XT_ERR_INVALID,
                          f"FastTensor::rmsnorm weight size mismatch: expected {n}, got {weight.numel()}")
-    x2 = x.reshape(-1, n).contiguous()
+    x2 = _rows(x).contiguous()
     y = out if out is not None else torch.empty_like(x2)
     _check(_lib.xt_rms_norm(_dev_ptr(x2, torch.float32, "x"),
                             _dev_ptr(weight.contiguous(), torch.float32, "weight"), x2.shape[0], n,
@@ -675,7 +694,7 @@ def mlp_q(gate, up, down, q, inv, norm_w=None, eps=1e-5, use_silu=False,
     """xt_ternary_mlp_q: fused_mlp_all on every row of q [M, in_dim] i8."""
     torch = _torch()
     _mlp_check(gate, up, down, q.shape[-1])
-    q2 = q.reshape(-1, q.shape[-1]).contiguous()
+    q2 = _rows(q).contiguous()
     M = q2.shape[0]
     y = out if out is not None else torch.empty((M, down.out_dim), dtype=torch.float32,
                                                 device=q.device)
@@ -693,7 +712,7 @@ def mlp_f32(gate, up, down, x, norm_w=None, eps=1e-5, use_silu=False, mode=XT_QU
     """xt_ternary_mlp_f32: Mlp::forward for x [M, in_dim] f32."""
     torch = _torch()
     _mlp_check(gate, up, down, x.shape[-1])
-    x2 = x.reshape(-1, x.shape[-1]).contiguous()
+    x2 = _rows(x).contiguous()
     M = x2.shape[0]
     y = out if out is not None else torch.empty((M, down.out_dim), dtype=torch.float32,
                                                 device=x.device)
@@ -714,7 +733,7 @@ def _multi(ws, ys):
 
 def linear_multi_f32(ws, x, mode=XT_QUANT_AVX512, stream=None, outs=None):
     torch = _torch()
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = _rows(x)
     M = x2.shape[0]
     ys = outs if outs is not None else [torch.empty((M, w.out_dim), dtype=torch.float32,
                                                     device=x.device) for w in ws]
@@ -726,7 +745,7 @@ def linear_multi_f32(ws, x, mode=XT_QUANT_AVX512, stream=None, outs=None):
 
 def linear_multi_q(ws, q, inv, stream=None):
     torch = _torch()
-    q2 = q.reshape(-1, q.shape[-1])
+    q2 = _rows(q)
     M = q2.shape[0]
     ys = [torch.empty((M, w.out_dim), dtype=torch.float32, device=q.device) for w in ws]
     harr, yarr = _multi(ws, ys)
@@ -761,11 +780,11 @@ class Stack:
                 raise XternError(XT_ERR_INVALID, f"op {i}: need 1..4 weights and as many outputs")
             o = arr[i]
             o.n = len(ws)
-            o.x = _dev_ptr(x, torch.float32, "x").value
+            o.x = _dev_ptr(x, torch.float32, "x")
             o.dep = -1 if dep is None else int(dep)
             for p, (w, y) in enumerate(zip(ws, ys)):
                 o.w[p] = w.handle.value
-                o.y[p] = _dev_ptr(y, torch.float32, "y").value
+                o.y[p] = _dev_ptr(y, torch.float32, "y")
             self._keep += [x] + list(ys) + list(ws)
         h = ctypes.c_void_p()
         _check(_lib.xt_stack_create(arr, len(ops), M, mode | self._PLANS[plan], ctypes.byref(h)))

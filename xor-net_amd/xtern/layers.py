@@ -174,7 +174,8 @@ class TernaryLinear:
         """layers.rs:262-313: per-row absmax i8 quantisation, ternary product,
         y = (f32)dot * inv_scale[row] * w_scales[o]."""
         shape = self._out_shape(xs)
-        return linear_f32(self.weights, xs.contiguous(), mode=mode).reshape(shape)
+        y = linear_f32(self.weights, xs.contiguous(), mode=mode)
+        return y if xs.dim() == 2 else y.reshape(shape)
 
     def forward_with_quantized(self, xs, quantized_in, inv_scale):
         """layers.rs:315-345 (for any number of rows): `xs` only supplies the
@@ -263,7 +264,8 @@ class _IntLinear:
 
     def forward(self, xs, mode=XT_QUANT_AVX512):
         shape = self._check(xs)
-        return linear_f32(self.weights, xs.contiguous(), mode=mode).reshape(shape)
+        y = linear_f32(self.weights, xs.contiguous(), mode=mode)
+        return y if xs.dim() == 2 else y.reshape(shape)
 
     def forward_with_quantized(self, xs, quantized_in, inv_scale):
         import torch
@@ -318,7 +320,7 @@ class Mlp:
         y = mlp_f32(self.c_fc1.weights, self.c_fc2.weights, self.c_proj.weights, x.contiguous(),
                     norm_w=n.weight if n is not None else None, eps=n.eps if n is not None else 0.0,
                     use_silu=self.hidden_act == "silu", mode=mode)
-        return y.reshape(tuple(x.shape[:-1]) + (self.c_proj.out_dim,))
+        return y if x.dim() == 2 else y.reshape(tuple(x.shape[:-1]) + (self.c_proj.out_dim,))
 
     def weight_bytes(self):
         """mlp.rs:140-143: packed weight bytes of the three projections."""
