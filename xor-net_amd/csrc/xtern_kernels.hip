@@ -154,6 +154,67 @@ __global__ __launch_bounds__(256) void rowsum_kernel(const int8_t* __restrict__ 
     if (threadIdx.x == 0) rowsum[m] = sum;
 }
 
+// The same for rows of any length and 4-byte alignment (ldx, K or the buffers
+// not multiples of 4): the pieces of four are loaded and stored at whatever
+// alignment they have (gfx950 takes it), the last K % 4 elements one by one.
+// quantize_kernel reads such a row twice, one element per lane and step:
+// 37 x 1003 4.3 -> 3.3 us, 300 x 7001 15.2 -> 5.1, 2048 x 3203 14.8 -> 11.2.
+typedef float uf4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t uu32 __attribute__((aligned(1)));
+template <int NV, int NT>
+__global__ __launch_bounds__(NT) void quantize_any_kernel(const float* __restrict__ x, int64_t ldx, int K,
+                                                          int8_t* __restrict__ q, int ldq,
+                                                          float* __restrict__ inv,
+                                                          int32_t* __restrict__ rowsum, int mode) {
+    __shared__ float sm_f[NT / 64];
+    __shared__ int sm_i[NT / 64];
+    const int m = blockIdx.x;
+    const float* xr = x + (size_t)m * ldx;
+    int8_t* qr = q + (size_t)m * ldq;
+    const int K4 = K >> 2, rem = K & 3;  // K4 >= 1
+    float v[NV][4], tail = 0.0f;
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+        const int i = min((int)threadIdx.x + u * NT, K4 - 1);
+        const uf4 t = *reinterpret_cast<const uf4*>(xr + 4 * i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[u][e] = t[e];
+    }
+    if ((int)threadIdx.x < rem) tail = xr[4 * K4 + threadIdx.x];
+    float mx = fabsf(tail);
+#pragma unroll
+    for (int u = 0; u < NV; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mx = fmaxf(mx, fabsf(v[u][e]));  // (a clamped piece: its own maximum again)
+    mx = block_reduce<NT / 64>(mx, MaxOp(), sm_f);
+    const float scale = (mx > 0.0f) ? __fdiv_rn(127.0f, mx) : 1.0f;
+    const float invs = (mx > 0.0f) ? __fdiv_rn(mx, 127.0f) : 1.0f;
+    const int kmain = (K / 16) * 16;
+    int sum = 0;
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+        const int i = threadIdx.x + u * NT;
+        if (i >= K4) continue;
+        int b[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) b[t] = quant_one(v[u][t], scale, mode, 4 * i + t < kmain);
+        sum += b[0] + b[1] + b[2] + b[3];
+        *reinterpret_cast<uu32*>(qr + 4 * i) = (uint32_t)(b[0] & 255) | ((uint32_t)(b[1] & 255) << 8) |
+                                               ((uint32_t)(b[2] & 255) << 16) | ((uint32_t)(b[3] & 255) << 24);
+    }
+    if ((int)threadIdx.x < rem) {  // (past the last 16 elements: the scalar tail's rounding)
+        const int b = quant_one(tail, scale, mode, false);
+        sum += b;
+        qr[4 * K4 + threadIdx.x] = (int8_t)b;
+    }
+    for (int i = K + threadIdx.x; i < ldq; i += NT) qr[i] = 0;  // padding
+    if (rowsum) sum = block_reduce<NT / 64>(sum, AddOp(), sm_i);  // uniform: skipped when unused
+    if (threadIdx.x == 0) {
+        inv[m] = invs;
+        if (rowsum) rowsum[m] = sum;
+    }
+}
+
 hipError_t launch_quantize(const float* x, int64_t ldx, int M, int K, int8_t* q, int ldq,
                            float* inv, int32_t* rowsum, int mode, hipStream_t s) {
     if (M <= 0) return hipSuccess;
@@ -172,6 +233,20 @@ hipError_t launch_quantize(const float* x, int64_t ldx, int M, int K, int8_t* q,
         XT_QREG(2, 1024)
         XT_QREG(4, 1024)
 #undef XT_QREG
+    }
+    if (K >= 4 && K <= 16384 && (uintptr_t)x % 4 == 0) {
+#define XT_QANY(NV_, NT_)                                                                        \
+    if (K / 4 <= NT_ * NV_) {                                                                    \
+        hipLaunchKernelGGL((quantize_any_kernel<NV_, NT_>), dim3(M), dim3(NT_), 0, s, x, ldx, K, q, \
+                           ldq, inv, rowsum, mode);                                              \
+        return hipGetLastError();                                                                \
+    }
+        XT_QANY(1, 256)
+        XT_QANY(2, 256)
+        XT_QANY(1, 1024)
+        XT_QANY(2, 1024)
+        XT_QANY(4, 1024)
+#undef XT_QANY
     }
     hipLaunchKernelGGL(quantize_kernel, dim3(M), dim3(256), 0, s, x, ldx, K, q, ldq, inv, rowsum,
                        mode);
