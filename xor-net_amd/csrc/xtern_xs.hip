@@ -47,8 +47,11 @@ __device__ __forceinline__ v4i xs_ld128(__amdgpu_buffer_rsrc_t r, unsigned off) 
     return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
 }
 
-// MT: token rows per launch (1, 4 or 16; M <= MT); NIT: block quads per
-// wave; W: waves per workgroup.
+// MT: token rows per launch (1, 4, 8 or 16; M <= MT); NIT: block quads per
+// wave; W: waves per workgroup.  The activation slice holds MT rows: a
+// workgroup of 8 waves takes 43 KiB of LDS at MT = 4 and 75 KiB at 16, so
+// three of them share a CU instead of two and hide more of the two dependent
+// load rounds (4096 -> 14336, M = 4: 15.0 -> 13.2 us; M = 8: 15.0 -> 14.1).
 template <int MT, int NIT, int W>
 __global__ __launch_bounds__(W * 64) void xs_gemv_kernel(const XsArgs a) {
     constexpr int kXsWaves = W;
@@ -57,7 +60,7 @@ __global__ __launch_bounds__(W * 64) void xs_gemv_kernel(const XsArgs a) {
     // MT > 1: per wave, the quad's expanded weights [block][row][16-byte
     // piece] and activation rows [token][piece] (one piece of padding per row)
     __shared__ v4i wsl[MT > 1 ? kXsWaves : 1][4][16][4];
-    __shared__ v4i asl[MT > 1 ? kXsWaves : 1][16][17];
+    __shared__ v4i asl[MT > 1 ? kXsWaves : 1][MT > 1 ? MT : 1][17];
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int j = lane & 15, bq = lane >> 4;
@@ -153,16 +156,17 @@ __global__ __launch_bounds__(W * 64) void xs_gemv_kernel(const XsArgs a) {
                     acc[0] = __builtin_amdgcn_sdot4((int)wd[4 * u + d], x1[it][u][d], acc[0], false);
         } else {
             // The quad's 4 x 64 columns: the expanded weights (lane order,
-            // row j of block bq) and the activation rows (4-row loads:
+            // row j of block bq) and the MT activation rows (4-row loads:
             // token 4u + lane / 16, piece lane % 16) go through the wave's
             // LDS slices, then one MFMA per block takes 16 tokens x 16 rows
             // x 64 columns.  (A wave's LDS accesses complete in order: no
             // barrier.)
             const int q0 = wave + it * kXsWaves;  // the quad
             const bool qlive = 4 * q0 < nb;
-            v4i xa[4];
+            constexpr int U = MT > 4 ? MT / 4 : 1;  // loads of 4 rows
+            v4i xa[U];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
+            for (int u = 0; u < U; ++u) {
                 const int m = 4 * u + (lane >> 4);
                 xa[u] = xs_ld128(qr, (qlive && m < M) ? (unsigned)m * (unsigned)a.ldq + (unsigned)q0 * 256u +
                                                             (unsigned)(lane & 15) * 16u
@@ -172,11 +176,11 @@ __global__ __launch_bounds__(W * 64) void xs_gemv_kernel(const XsArgs a) {
             for (int p = 0; p < 4; ++p)
                 wsl[wave][bq][j][p] = v4i{(int)wd[4 * p], (int)wd[4 * p + 1], (int)wd[4 * p + 2], (int)wd[4 * p + 3]};
 #pragma unroll
-            for (int u = 0; u < 4; ++u) asl[wave][4 * u + (lane >> 4)][lane & 15] = xa[u];
+            for (int u = 0; u < U; ++u) asl[wave][4 * u + (lane >> 4)][lane & 15] = xa[u];
             __asm__ volatile("" ::: "memory");
 #pragma unroll
             for (int b = 0; b < 4; ++b)
-                macc = mfma(asl[wave][j][4 * b + g], wsl[wave][b][j][g], macc);
+                macc = mfma(asl[wave][j & (MT - 1)][4 * b + g], wsl[wave][b][j][g], macc);  // (rows >= MT: not kept)
             __asm__ volatile("" ::: "memory");
         }
     }
@@ -189,7 +193,8 @@ __global__ __launch_bounds__(W * 64) void xs_gemv_kernel(const XsArgs a) {
     } else {
         // lane (g, j): tokens 4g + r of row j
 #pragma unroll
-        for (int rr = 0; rr < 4; ++rr) red[wave][4 * g + rr][j] = macc[rr];
+        for (int rr = 0; rr < 4; ++rr)
+            if (4 * g + rr < MT) red[wave][4 * g + rr][j] = macc[rr];
     }
     __syncthreads();
     if (t < 16 * MT) {
@@ -234,6 +239,8 @@ int xs_max_rows() { return 16; }
 
 hipError_t launch_xs_gemv(const XsArgs& a, hipStream_t s) {
     if (a.M <= 1) return launch_mt<1>(a, s);
+    if (a.M <= 4) return launch_mt<4>(a, s);
+    if (a.M <= 8) return launch_mt<8>(a, s);
     return launch_mt<16>(a, s);
 }
 
