@@ -829,10 +829,10 @@ bool gemv_fits(int fmt, int M, int nch, int waves, int ncw) {
 // v_perm_b32 (code 0 -> -1, 1 -> 0, 2 -> +1, 3 -> 0), so no activation row
 // sum is needed.  Waves are summed through LDS once at the end.
 
-// FUSED: the kernel quantises the f32 rows a.x itself (quantization.rs:95-195,
-// as quantize_kernel): each lane reads its pieces as f32, the per-token
-// absmax goes through the waves' shuffles and LDS (one barrier), then each
-// lane quantises its own pieces.  No separate quantiser launch.
+// FUSED: the kernel quantises the one f32 row a.x itself (quantization.rs:95-195,
+// as quantize_kernel): each lane reads its pieces as f32, the row's absmax
+// goes through the waves' shuffles and LDS (one barrier), then each lane
+// quantises its own pieces.  No separate quantiser launch.
 // AM > 0 (M <= AM, q given): the wave's activation bytes (rows < M of its
 // chunks, 256 / 320 bytes each) are loaded once, one distinct 16-byte piece
 // per lane, passed through a wave-private LDS slice and read back as MFMA
@@ -853,6 +853,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv2_kernel(const MMArgs a) {
     __shared__ v4i red[WAVES][RG][64];
     __shared__ v4i aslice[WAVES][AM == 16 ? 16 * 17 : (AM > 0 ? AM * APS : 1)];
     __shared__ unsigned tmax[WAVES][16];
+    __shared__ __align__(16) unsigned qrow[FUSED ? WAVES : 1][FUSED ? NCW : 1][FUSED ? CH / 4 : 4];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int g = lane >> 4;
@@ -970,112 +971,23 @@ __global__ __launch_bounds__(WAVES * 64) void gemv2_kernel(const MMArgs a) {
             for (int s = 0; s < STEPS; ++s) av[t][s] = ld_cached(arow + (size_t)c * CH + s * 64);
         }
     } else {
-        // Cooperative quantisation: thread t takes float4 pieces t, t + NT,
-        // ... of the M x K rows (K % 4 == 0, so a piece never straddles two
-        // rows), gathers each token's absmax through LDS, quantises its
-        // pieces into the A-operand stage [chunk][step][g][token 0..15][16 B],
-        // and after a barrier every lane reads its fragments.  Stage bytes of
-        // columns >= K are never written; their weights are padding code 1,
-        // which decodes to 0.
-        extern __shared__ __align__(16) uint8_t stage[];
         const int K = a.K;
-        constexpr int NT = WAVES * 64;
-        const int n4 = (M * K) >> 2;
+        const int n4 = K >> 2;
         // One row: lane l of wave w loads float4 piece l of each chunk the
         // wave multiplies (chunks w + t WAVES), and for Pack5's 80-piece
         // chunks also piece 64 + l (l < 16), so every lane finds its A
         // fragment in the packed bytes of four lanes of its own wave
-        // (ds_bpermute, no LDS stage); the row maximum comes from per-wave
+        // (its LDS row, no stage); the row maximum comes from per-wave
         // maxima (no atomics, so no clearing barrier).  One barrier in all.
         constexpr int PPC = CH / 4;  // float4 pieces per chunk: 64 or 80
-        bool one_pass = false;
-        if constexpr (FMT == XT_PACK4 || FMT == XT_PACK5) one_pass = M == 1;
-        if (one_pass) {
-            float4 x0[NCW], x1[NCW];
+        float4 x0[NCW], x1[NCW];
 #pragma unroll
-            for (int t = 0; t < NCW; ++t) {
-                const int f = (wave + t * WAVES) * PPC + lane;
-                x0[t] = x1[t] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if (f < n4) x0[t] = *reinterpret_cast<const float4*>(a.x + 4 * f);
-                if constexpr (PPC > 64)
-                    if (lane < PPC - 64 && f + 64 < n4) x1[t] = *reinterpret_cast<const float4*>(a.x + 4 * (f + 64));
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int t = 0; t < NCW; ++t) {
-                const int c = min(wave + t * WAVES, nch - 1);
-#pragma unroll
-                for (int r = 0; r < RG; ++r)
-#pragma unroll
-                    for (int u = 0; u < TPC; ++u)
-                        wv[t][r][u] = ld_stream(wsrc[r] + ((size_t)c * TPC + u) * kTileBytes);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            // (non-negative floats order as their bit patterns; NaN is ignored)
-            auto amax = [](float4 v) { return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))); };
-            float mx = 0.0f;
-#pragma unroll
-            for (int t = 0; t < NCW; ++t) mx = fmaxf(mx, fmaxf(amax(x0[t]), amax(x1[t])));
-            const int wm = wave_reduce_bits(__float_as_int(mx), [](int p, int q) {
-                return __float_as_int(fmaxf(__int_as_float(p), __int_as_float(q)));
-            });
-            if (lane == 0) tmax[wave][0] = (unsigned)wm;
-            __syncthreads();
-            unsigned mb = 0u;
-#pragma unroll
-            for (int w = 0; w < WAVES; ++w) mb = max(mb, tmax[w][0]);
-            const float rmx = __uint_as_float(mb);
-            const float scale = (rmx > 0.0f) ? __fdiv_rn(127.0f, rmx) : 1.0f;
-            const float iv = (rmx > 0.0f) ? __fdiv_rn(rmx, 127.0f) : 1.0f;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) invr[r] = iv;
-            const int kmain = (K / 16) * 16;
-            unsigned w4[NCW], w5[NCW];
-            auto pack = [&](auto mode_c) {
-                auto q4 = [&](float4 v, int f) {
-                    const int col = 4 * f;
-                    const float e4[4] = {v.x, v.y, v.z, v.w};
-                    unsigned r = 0;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        r |= (unsigned)(quant_one(e4[e], scale, decltype(mode_c)::value, col + e < kmain) & 255)
-                             << (8 * e);
-                    return f < n4 ? r : 0u;  // columns past K: zero activations
-                };
-#pragma unroll
-                for (int t = 0; t < NCW; ++t) {
-                    const int f = (wave + t * WAVES) * PPC + lane;
-                    w4[t] = q4(x0[t], f);
-                    w5[t] = PPC > 64 ? q4(x1[t], f + 64) : 0u;
-                }
-            };
-            if (a.mode == XT_QUANT_AVX512) pack(std::integral_constant<int, XT_QUANT_AVX512>{});
-            else pack(std::integral_constant<int, XT_QUANT_SCALAR>{});
-            // lane (g, j) of step s takes chunk pieces 16 s + 4 g + d: lanes
-            // 0..63 of the first packed value, then lanes 0..15 of the second
-#pragma unroll
-            for (int t = 0; t < NCW; ++t)
-#pragma unroll
-                for (int st = 0; st < STEPS; ++st)
-#pragma unroll
-                    for (int d = 0; d < 4; ++d) {
-                        const int idx = 16 * st + 4 * g + d;
-                        av[t][st][d] = st < 4 ? __builtin_amdgcn_ds_bpermute(idx << 2, (int)w4[t])
-                                              : __builtin_amdgcn_ds_bpermute((idx - 64) << 2, (int)w5[t]);
-                    }
-        } else {
-        if (threadIdx.x < 16) tmax[0][threadIdx.x] = 0u;
-        // The f32 pieces are loaded before the weights: loads return in
-        // order, so the quantiser then waits for its own loads only and runs
-        // while the weights are in flight.
-        float4 xv[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int f = threadIdx.x + u * NT;
-            if (f < n4) {
-                const int m = (4 * f) / K, col = 4 * f - m * K;
-                xv[u] = *reinterpret_cast<const float4*>(a.x + (size_t)m * a.ldx + col);
-            }
+        for (int t = 0; t < NCW; ++t) {
+            const int f = (wave + t * WAVES) * PPC + lane;
+            x0[t] = x1[t] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (f < n4) x0[t] = *reinterpret_cast<const float4*>(a.x + 4 * f);
+            if constexpr (PPC > 64)
+                if (lane < PPC - 64 && f + 64 < n4) x1[t] = *reinterpret_cast<const float4*>(a.x + 4 * (f + 64));
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1088,66 +1000,63 @@ __global__ __launch_bounds__(WAVES * 64) void gemv2_kernel(const MMArgs a) {
                     wv[t][r][u] = ld_stream(wsrc[r] + ((size_t)c * TPC + u) * kTileBytes);
         }
         __builtin_amdgcn_sched_barrier(0);
-        __syncthreads();  // tmax cleared
         // (non-negative floats order as their bit patterns; NaN is ignored)
+        auto amax = [](float4 v) { return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))); };
+        float mx = 0.0f;
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int f = threadIdx.x + u * NT;
-            const int f0 = wave * 64 + u * NT;  // first piece of this wave
-            if (f0 >= n4) continue;
-            const float mx = f < n4 ? fmaxf(fmaxf(fabsf(xv[u].x), fabsf(xv[u].y)),
-                                            fmaxf(fabsf(xv[u].z), fabsf(xv[u].w)))
-                                    : 0.0f;
-            const int m0 = (4 * f0) / K, m1 = (4 * min(f0 + 63, n4 - 1)) / K;
-            if (m0 == m1) {  // the wave's pieces lie in one row: one atomic per wave
-                const int wm = wave_reduce_bits(__float_as_int(mx), [](int x, int y) {
-                    return __float_as_int(fmaxf(__int_as_float(x), __int_as_float(y)));
-                });
-                if (lane == 0) atomicMax(&tmax[0][m0], (unsigned)wm);
-            } else if (f < n4) {
-                atomicMax(&tmax[0][(4 * f) / K], __float_as_uint(mx));
-            }
-        }
+        for (int t = 0; t < NCW; ++t) mx = fmaxf(mx, fmaxf(amax(x0[t]), amax(x1[t])));
+        const int wm = wave_reduce_bits(__float_as_int(mx), [](int p, int q) {
+            return __float_as_int(fmaxf(__int_as_float(p), __int_as_float(q)));
+        });
+        if (lane == 0) tmax[wave][0] = (unsigned)wm;
         __syncthreads();
+        unsigned mb = 0u;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) mb = max(mb, tmax[w][0]);
+        const float rmx = __uint_as_float(mb);
+        const float scale = (rmx > 0.0f) ? __fdiv_rn(127.0f, rmx) : 1.0f;
+        const float iv = (rmx > 0.0f) ? __fdiv_rn(rmx, 127.0f) : 1.0f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) invr[r] = iv;
         const int kmain = (K / 16) * 16;
-        // (the rounding mode is chosen once, so that only one quantiser's
-        // code runs through the unrolled loop)
-        auto quant_pieces = [&](auto mode_c) {
+        unsigned w4[NCW], w5[NCW];
+        auto pack = [&](auto mode_c) {
+            auto q4 = [&](float4 v, int f) {
+                const int col = 4 * f;
+                const float e4[4] = {v.x, v.y, v.z, v.w};
+                unsigned r = 0;
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int f = threadIdx.x + u * NT;
-                if (f < n4) {
-                    const int m = (4 * f) / K, col = 4 * f - m * K;
-                    const float rmx = __uint_as_float(tmax[0][m]);
-                    const float scale = (rmx > 0.0f) ? __fdiv_rn(127.0f, rmx) : 1.0f;
-                    const float e4[4] = {xv[u].x, xv[u].y, xv[u].z, xv[u].w};
-                    unsigned w4 = 0;
+                for (int e = 0; e < 4; ++e)
+                    r |= (unsigned)(quant_one(e4[e], scale, decltype(mode_c)::value, col + e < kmain) & 255)
+                         << (8 * e);
+                return f < n4 ? r : 0u;  // columns past K: zero activations
+            };
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        w4 |= (unsigned)(quant_one(e4[e], scale, decltype(mode_c)::value, col + e < kmain) & 255)
-                              << (8 * e);
-                    const int c = col / CH, r = col - c * CH, st = r >> 6, gg = (r >> 4) & 3;
-                    *reinterpret_cast<unsigned*>(stage + ((((c * STEPS + st) * 4 + gg) * 16 + m) << 4) + (col & 15)) = w4;
-                }
+            for (int t = 0; t < NCW; ++t) {
+                const int f = (wave + t * WAVES) * PPC + lane;
+                w4[t] = q4(x0[t], f);
+                w5[t] = PPC > 64 ? q4(x1[t], f + 64) : 0u;
             }
         };
-        if (a.mode == XT_QUANT_AVX512) quant_pieces(std::integral_constant<int, XT_QUANT_AVX512>{});
-        else quant_pieces(std::integral_constant<int, XT_QUANT_SCALAR>{});
-        __syncthreads();
+        if (a.mode == XT_QUANT_AVX512) pack(std::integral_constant<int, XT_QUANT_AVX512>{});
+        else pack(std::integral_constant<int, XT_QUANT_SCALAR>{});
+        // The chunk's packed bytes through the wave's LDS row: lane (g, j)
+        // of step s reads pieces 16 s + 4 g .. + 3, the same 16 bytes for
+        // every j (one write and four broadcast reads per chunk against
+        // 16 ds_bpermute: 2560 -> 640 4.32 -> 3.86 us, 6912 -> 2560 5.81 ->
+        // 5.64).  A wave's LDS accesses complete in order: no barrier.
 #pragma unroll
         for (int t = 0; t < NCW; ++t) {
-            const int c = min(wave + t * WAVES, nch - 1);
+            qrow[wave][t][lane] = w4[t];
+            if constexpr (PPC > 64)
+                if (lane < PPC - 64) qrow[wave][t][64 + lane] = w5[t];
+        }
+        __asm__ volatile("" ::: "memory");
 #pragma unroll
-            for (int s = 0; s < STEPS; ++s)
-                av[t][s] = *reinterpret_cast<const v4i*>(stage + ((((c * STEPS + s) * 4 + g) * 16 + j) << 4));
-        }
-        // inverse scales of tokens 4g + r (wave 0 finishes)
+        for (int t = 0; t < NCW; ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float x2 = __uint_as_float(tmax[0][min(4 * g + r, 15)]);
-            invr[r] = (x2 > 0.0f) ? __fdiv_rn(x2, 127.0f) : 1.0f;
-        }
-        }
+            for (int st = 0; st < STEPS; ++st)
+                av[t][st] = *reinterpret_cast<const v4i*>(&qrow[wave][t][16 * st + 4 * g]);
     }
     v4i acc[RG][STEPS];
 #pragma unroll
@@ -1156,7 +1065,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemv2_kernel(const MMArgs a) {
         for (int s = 0; s < STEPS; ++s) acc[r][s] = v4i{0, 0, 0, 0};
 #pragma unroll
     for (int t = 0; t < NCW; ++t) {
-        const bool live = wave + t * WAVES < nch;
+        // (A rows >= M only reach sums that are not stored, and the fused
+        // quantiser's chunks past the row are zeros: no select there.  Skipping
+        // such chunks, or leaving the select to them alone, was slower at
+        // M = 16, 14336 -> 4096: 8.0 -> 8.6 us)
+        const bool live = FUSED || wave + t * WAVES < nch;
 #pragma unroll
         for (int r = 0; r < RG; ++r) {
             if constexpr (FMT == XT_PACK5) {
@@ -1176,7 +1089,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv2_kernel(const MMArgs a) {
                         E[d] = pE & 0x00ff00ff;
                         O[d] = pO & 0x00ff00ff;
                     }
-                    const v4i x = (live && j < M) ? av[t][s] : v4i{0, 0, 0, 0};
+                    const v4i x = FUSED || (live && j < M) ? av[t][s] : v4i{0, 0, 0, 0};
                     acc[r][s] = mfma(x, b, acc[r][s]);
                 }
             } else {
@@ -1198,7 +1111,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemv2_kernel(const MMArgs a) {
 #pragma unroll
                         for (int d = 0; d < 4; ++d) b[d] = signed_codes(b[d]);
                     }
-                    const v4i x = (live && j < M) ? av[t][s] : v4i{0, 0, 0, 0};
+                    const v4i x = FUSED || (live && j < M) ? av[t][s] : v4i{0, 0, 0, 0};
                     acc[r][s] = mfma(x, b, acc[r][s]);
                 }
             }
@@ -1246,8 +1159,7 @@ static int gemv2_rg_for(int fmt, int nch, int ngroups) {
     return 1;
 }
 
-// Waves of the staging-free GEMV for nch chunks, and the most f32 elements
-// (M * K) its fused quantiser takes: 8 float4 per thread.
+// Waves of the staging-free GEMV for nch chunks.
 static int gemv2_waves(int nch) {
     for (int w : {4, 8, 10, 16})
         if (nch <= w) return w;
@@ -1255,16 +1167,15 @@ static int gemv2_waves(int nch) {
     // chunks per wave)
     return (nch <= 28 || (nch > 32 && nch <= 42) || (nch > 48 && nch <= 56)) ? 14 : 16;
 }
-// LDS of the fused GEMV: the A stage (1 KiB per k-step) plus the static
-// cross-wave sums and maxima; it must fit the 160 KiB of a CU.
-static size_t gemv2_fused_lds(int nch, int steps, int rg) {
-    const int w = gemv2_waves(nch);
-    return (size_t)nch * steps * 1024 + (size_t)w * rg * 64 * 16 + (size_t)w * 16 * 4;
-}
-constexpr size_t kLdsBytes = 160 * 1024;
+// Longest f32 row the fused GEMV takes: rows of at most about 36 (Pack5 28)
+// chunks, so that the row's registers and the workgroups' repeated reads of
+// it stay small; longer rows take the quantiser launch.  (Every workgroup
+// quantises the whole row: 4096 -> 14336, 448 workgroups, 10.1 us fused vs
+// 8.6 with the launch.)
 int gemv2_fused_max(int fmt, int nch, int rg) {
-    if (nch > 64 || gemv2_fused_lds(nch, fmt == XT_PACK5 ? 5 : 4, rg) > kLdsBytes) return 0;
-    return gemv2_waves(nch) * 64 * 32;
+    const int steps = fmt == XT_PACK5 ? 5 : 4, w = gemv2_waves(nch);
+    if (nch > 64 || nch * steps * 1024 + w * rg * 64 * 16 + w * 16 * 4 > 160 * 1024) return 0;
+    return w * 64 * 32;
 }
 
 // Quantised rows given: the activation pieces through a wave-private LDS
@@ -1332,22 +1243,14 @@ static hipError_t launch_gemv2_int(const MMArgs& a, int ntiles, hipStream_t s) {
 template <int RG>
 static hipError_t launch_gemv2_rg(int fmt, const MMArgs& a, int ntiles, hipStream_t s) {
     const int nch = a.nch;
-    // fused rows: at most 8 float4 per thread, A stage of 1 KiB per k-step
-    const int steps = fmt == XT_PACK5 ? 5 : 4;
-    const size_t stage = (size_t)nch * steps * 1024;
-    if (a.x && gemv2_fused_lds(nch, steps, RG) > kLdsBytes) return hipErrorInvalidValue;
+    if (a.x && (a.M != 1 || a.K > gemv2_fused_max(fmt, nch, RG))) return hipErrorInvalidValue;
 #define XT_GV2(W_, NCW_)                                                                         \
     if (nch <= W_ * NCW_) {                                                                      \
         if (a.x) {                                                                               \
-            if ((size_t)a.M * a.K > (size_t)W_ * 64 * 32) {                                   \
-                return hipErrorInvalidValue; /* fused rows: 8 float4 per thread */               \
-            } else if (fmt == XT_PACK5) {                                                        \
-                hipLaunchKernelGGL((gemv2_kernel<XT_PACK5, W_, NCW_, true, RG>), dim3(ntiles), dim3(W_ * 64), a.M == 1 ? 0 : stage, s, a); \
-            } else {                                                                             \
-                /* one row in one pass: no LDS stage */                                          \
-                const size_t st_ = a.M == 1 ? 0 : stage;                                    \
-                hipLaunchKernelGGL((gemv2_kernel<XT_PACK4, W_, NCW_, true, RG>), dim3(ntiles), dim3(W_ * 64), st_, s, a); \
-            }                                                                                    \
+            if (fmt == XT_PACK5)                                                                 \
+                hipLaunchKernelGGL((gemv2_kernel<XT_PACK5, W_, NCW_, true, RG>), dim3(ntiles), dim3(W_ * 64), 0, s, a);\
+            else                                                                                 \
+                hipLaunchKernelGGL((gemv2_kernel<XT_PACK4, W_, NCW_, true, RG>), dim3(ntiles), dim3(W_ * 64), 0, s, a);\
         } else if (fmt == XT_PACK5) {                                                            \
             return launch_gemv2_am<XT_PACK5, W_, NCW_, RG>(a, ntiles, s);                      \
         } else if (fmt == XT_INT8) {                                                             \
