@@ -1391,8 +1391,9 @@ int int_gemv_waves(int fmt, int mb, int nch) {
 namespace {
 // Shapes of a product with more than 16 rows, and what one workgroup of each
 // costs per chunk of K: `first` when it has its CU to itself, `rest` for each
-// further workgroup of the CU, `gap` once per further workgroup (microseconds;
-// `unit`: K is taken in rounds of so many chunks).  Fitted to launch-to-launch
+// further workgroup of the CU, `gap` once per further workgroup (its start and
+// epilogue, as far as they are not hidden; microseconds; `unit`: K is taken
+// in rounds of so many chunks).  Fitted to launch-to-launch
 // times on MI355X over M = 20 .. 2048 and K, N = 512 .. 14336 (weights
 // streamed from memory); with a few launches more or less per CU the totals
 // are within about 15 % of the measured ones, and where two shapes come out
@@ -1411,8 +1412,8 @@ struct GemmShape {
 const GemmShape kShapes4[] = {
     {1, 2, 4, 4, 0, 0.170f, 0.170f, 1.0f, 1},  {1, 4, 8, 2, 0, 0.160f, 0.160f, 1.2f, 8},
     {1, 5, 8, 2, 0, 0.190f, 0.190f, 1.2f, 8},  {1, 8, 8, 2, 0, 0.245f, 0.245f, 1.2f, 8},
-    {2, 8, 4, 1, 4, 0.330f, 0.270f, 0.0f, 1},  {4, 8, 4, 1, 4, 0.480f, 0.450f, 0.0f, 1},
-    {4, 16, 4, 1, 4, 0.850f, 0.830f, 0.0f, 1}, {8, 16, 4, 1, 4, 1.570f, 1.450f, 0.0f, 1},
+    {2, 8, 4, 1, 4, 0.330f, 0.270f, 0.45f, 1}, {4, 8, 4, 1, 4, 0.480f, 0.450f, 0.6f, 1},
+    {4, 16, 4, 1, 4, 0.850f, 0.830f, 0.7f, 1}, {8, 16, 4, 1, 4, 1.570f, 1.450f, 1.5f, 1},
 };
 // Pack5 (the base-3 decode is 24 vector instructions per 16 weights against
 // 9, so shapes that decode a weight once for 128 tokens pay earlier): 3200 ->
@@ -1422,8 +1423,8 @@ const GemmShape kShapes4[] = {
 const GemmShape kShapes5[] = {
     {1, 2, 4, 4, 0, 0.290f, 0.160f, 0.0f, 1}, {1, 4, 8, 2, 0, 0.270f, 0.200f, 0.0f, 8},
     {1, 5, 8, 2, 0, 0.310f, 0.220f, 0.0f, 8}, {1, 5, 16, 1, 0, 0.275f, 0.360f, 0.0f, 16},
-    {2, 8, 4, 1, 4, 0.650f, 0.500f, 0.0f, 1}, {4, 8, 4, 1, 4, 0.800f, 0.680f, 0.0f, 1},
-    {8, 8, 4, 1, 4, 1.300f, 1.450f, 0.0f, 1}, {8, 16, 8, 1, 4, 2.000f, 2.350f, 0.0f, 1},
+    {2, 8, 4, 1, 4, 0.650f, 0.500f, 0.8f, 1}, {4, 8, 4, 1, 4, 0.800f, 0.620f, 2.2f, 1},
+    {8, 8, 4, 1, 4, 1.300f, 1.300f, 3.0f, 1}, {8, 16, 8, 1, 4, 2.000f, 2.200f, 3.5f, 1},
 };
 
 MMConfig choose_gemm(int fmt, int M, int ngroups, int nch) {
