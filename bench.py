@@ -918,7 +918,7 @@ def main():
     prod_ops = [2 * wl["M"] * s["N"] * s["K"] for s in wl["sets"]]
     ach = sum(prod_ops) / (sum(prod_ms) * 1e-3) / 1e12
     tr = recorded_traffic()
-    prod_tr = {k: v for k, v in (tr or {}).items() if k in ("gemm32s_up", "mm_down")}
+    prod_tr = {k: v for k, v in (tr or {}).items() if k in ("c1_up", "c1_down")}
     roof = {"bound": "mfma", "achieved": round(ach, 2), "peak": INT8_PEAK_TOPS,
             "unit": "TOPS", "frac": round(ach / INT8_PEAK_TOPS, 4),
             "traffic": (sum(prod_tr.values()) // len(prod_tr)) if prod_tr else None,
@@ -926,7 +926,7 @@ def main():
             "traffic_source": "profiles/pmc_traffic_c1.md (rocprofv3 --pmc FETCH_SIZE, "
                               "WRITE_SIZE of the same kernels, copy-calibrated; not measured "
                               "in this run)",
-            "kernel": "product launches (gemm32s_kernel up, mm_kernel down)",
+            "kernel": "product launches (gemmw_kernel up, mm_kernel down)",
             "us_per_launch": {s["name"]: round(m * 1e3, 3) for s, m in zip(wl["sets"], prod_ms)}}
 
     out = {"metric": "ternary GEMM int8 TOPS at M=128 (Pack4, BitNet-2B up+down)",
