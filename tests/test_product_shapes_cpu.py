@@ -1,0 +1,48 @@
+"""The shape rule of products with more than 16 rows (choose_config, a host
+function of libxtern.so), evaluated on the CPU: every shape it picks can be
+launched for the rows that a call may have."""
+import ctypes
+
+import pytest
+
+import xtern
+
+BLOCKS = 65535  # row blocks of a 16-token launch (its grid's y)
+
+
+class MMConfig(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int) for n in ("mb", "nb", "waves", "pf", "splitk", "kind")]
+
+
+def choose(fmt, M, groups, nch, rowsum=False):
+    f = xtern._lib["_ZN2xt13choose_configEiiiib"]
+    f.restype = MMConfig
+    f.argtypes = [ctypes.c_int] * 4 + [ctypes.c_bool]
+    return f(fmt, M, groups, nch, rowsum)
+
+
+@pytest.mark.parametrize("fmt,most", [(xtern.XT_PACK4, 18), (xtern.XT_XORSPARSE, 18), (xtern.XT_PACK5, 8)],
+                         ids=["pack4", "sparse", "pack5"])
+def test_rows_of_a_call_fit_the_chosen_launch(fmt, most, monkeypatch):
+    """Calls of up to 65535 x 32 rows are taken up to `most` chunks of K (up
+    to 65535 x 16 beyond): a 16-token shape must not be chosen above 65535
+    row blocks, whatever it is priced at."""
+    monkeypatch.delenv("XTERN_CONFIG", raising=False)
+    bad = []
+    for nch in list(range(1, most + 1)) + [most + 1, 40, 300]:
+        limit = BLOCKS * (32 if nch <= most else 16)
+        for M in (17, 1000, BLOCKS * 16 - 1, BLOCKS * 16, BLOCKS * 16 + 1, 1500001, BLOCKS * 32 - 31, BLOCKS * 32):
+            if M > limit:
+                continue
+            for groups in (1, 2, 3, 4, 5, 6, 8, 16, 432):
+                c = choose(fmt, M, groups, nch)
+                blocks = -(-M // (16 * c.mb))
+                if c.kind not in (0, 4) or (c.kind == 0 and blocks > BLOCKS):
+                    bad.append((M, groups, nch, c.kind, c.mb, c.nb))
+    assert not bad, f"{len(bad)}: {bad[:8]}"
+
+
+def test_narrow_pack5_of_a_million_rows():
+    assert choose(xtern.XT_PACK5, BLOCKS * 16, 2, 8).kind == 0  # (as priced, one block inside the limit)
+    assert choose(xtern.XT_PACK5, BLOCKS * 16 + 1, 2, 8).kind == 4
+    assert choose(xtern.XT_PACK5, 2097120, 6, 1).kind == 4

@@ -1433,8 +1433,11 @@ MMConfig choose_gemm(int fmt, int M, int ngroups, int nch) {
     MMConfig best;
     double best_cost = -1.0;
     auto take = [&](const GemmShape& g) {
-        const long tiles = (long)((M + 16 * g.mb - 1) / (16 * g.mb)) * ((ngroups + g.nb - 1) / g.nb);
+        const long blocks = (M + 16 * g.mb - 1) / (16 * g.mb);
+        const long tiles = blocks * ((ngroups + g.nb - 1) / g.nb);
         if (g.kind == 4 && (!wide || tiles > 0x7fffffff)) return;
+        // (mm_kernel's row blocks are its grid's y; gemmw_kernel's grid has x only)
+        if (g.kind == 0 && wide && blocks > 65535) return;
         const long n = (tiles + 255) / 256;  // workgroups of the busiest CU
         const double nc = (nch + g.unit - 1) / g.unit * g.unit;
         const double cost = g.first * nc + (double)(n - 1) * (g.rest * nc + g.gap);
