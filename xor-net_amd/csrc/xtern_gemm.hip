@@ -236,9 +236,14 @@ __global__ __launch_bounds__(64 * W, 2) void gemmw_kernel(const MMArgs a) {
     // chunk's.  In every k-step the next one's fragments are read and its
     // weights decoded between the MFMAs; the last step of a chunk first waits
     // for the next chunk and starts the loads of chunk c + D into the buffer
-    // and registers that chunk c no longer needs.
-    auto step = [&](int c, uint8_t* src, v4i (&w)[NW][2], const uint8_t* src2, v4i (&w2)[NW][2]) {
+    // and registers that chunk c no longer needs.  T >= 0: one of the last
+    // chunks, T of them before it, with no loads left to start: the wait must
+    // not count on any (weights that no later chunk multiplies are not even
+    // loaded), and of the loads in flight it counts the copies only.
+    auto step = [&](auto tail, int c, uint8_t* src, v4i (&w)[NW][2], const uint8_t* src2, v4i (&w2)[NW][2]) {
+        constexpr int T = decltype(tail)::value;
         constexpr int B = MW * NW, VALU = (FMT == XT_PACK5 ? 24 : 9) * NW, VM = LPT + 2 * NW;
+        constexpr bool more = T < D - 2;  // (T = D - 2: certainly the last)
 #pragma unroll
         for (int k = 0; k < 2 * STEPS; ++k) {
             const bool last = k + 1 == 2 * STEPS;
@@ -246,19 +251,20 @@ __global__ __launch_bounds__(64 * W, 2) void gemmw_kernel(const MMArgs a) {
             if (!last) {
                 read_f(src, (k + 1) / STEPS, (k + 1) % STEPS, av[(k + 1) & 1]);
                 decode(k + 1, w, bv[(k + 1) & 1]);
-            } else {
-                // (the loads of chunks c + 2 .. c + D - 1 may be in flight)
-                wait_copies<(D - 2) * VM>();
+            } else if constexpr (more) {
+                // (the loads of chunks c + 2 .. c + D - 1 - T may be in flight)
+                if constexpr (T < 0) wait_copies<(D - 2) * VM>();
+                else wait_copies<(D - 2 - T) * LPT>();
                 __builtin_amdgcn_sched_barrier(0);
                 read_f(src2, 0, 0, av[0]);
-                start(c + D, src, w);
+                if constexpr (T < 0) start(c + D, src, w);
                 decode(0, w2, bv[0]);
             }
 #pragma unroll
             for (int mb = 0; mb < MW; ++mb)
 #pragma unroll
                 for (int nb = 0; nb < NW; ++nb) acc[mb][nb] = mfma32(av[k & 1][mb], bv[k & 1][nb], acc[mb][nb]);
-            if constexpr (B == 8) if (last) interleave<0, B, MW, VM, (VALU + B - 1) / B + 4>();
+            if constexpr (B == 8 && T < 0) if (last) interleave<0, B, MW, VM, (VALU + B - 1) / B + 4>();
             if constexpr (B == 8) if (!last) interleave<0, B, MW, 0, (VALU + B - 1) / B>();
         }
     };
@@ -275,30 +281,32 @@ __global__ __launch_bounds__(64 * W, 2) void gemmw_kernel(const MMArgs a) {
     read_f(lds0, 0, 0, av[0]);
     decode(0, wv[0], bv[0]);
     int c = 0;
+    constexpr std::integral_constant<int, -1> loop{};
+    constexpr std::integral_constant<int, 0> tail0{};
     if constexpr (D == 2) {
         for (; c + 2 <= nch; c += 2) {
-            step(c, lds0, wv[0], lds1, wv[1]);
-            step(c + 1, lds1, wv[1], lds0, wv[0]);
+            step(loop, c, lds0, wv[0], lds1, wv[1]);
+            step(loop, c + 1, lds1, wv[1], lds0, wv[0]);
         }
-        if (c < nch) step(c, lds0, wv[0], lds1, wv[1]);
+        if (c < nch) step(tail0, c, lds0, wv[0], lds1, wv[1]);
     } else if constexpr (D == 3) {
         for (; c + 3 <= nch; c += 3) {
-            step(c, lds0, wv[0], lds1, wv[1]);
-            step(c + 1, lds1, wv[1], lds2, wv[2]);
-            step(c + 2, lds2, wv[2], lds0, wv[0]);
+            step(loop, c, lds0, wv[0], lds1, wv[1]);
+            step(loop, c + 1, lds1, wv[1], lds2, wv[2]);
+            step(loop, c + 2, lds2, wv[2], lds0, wv[0]);
         }
-        if (c < nch) step(c, lds0, wv[0], lds1, wv[1]);
-        if (c + 1 < nch) step(c + 1, lds1, wv[1], lds2, wv[2]);
+        if (c < nch) step(tail0, c, lds0, wv[0], lds1, wv[1]);
+        if (c + 1 < nch) step(std::integral_constant<int, 1>{}, c + 1, lds1, wv[1], lds2, wv[2]);
     } else {
         for (; c + 4 <= nch; c += 4) {
-            step(c, lds0, wv[0], lds1, wv[1]);
-            step(c + 1, lds1, wv[1], lds2, wv[2]);
-            step(c + 2, lds2, wv[2], lds3, wv[3]);
-            step(c + 3, lds3, wv[3], lds0, wv[0]);
+            step(loop, c, lds0, wv[0], lds1, wv[1]);
+            step(loop, c + 1, lds1, wv[1], lds2, wv[2]);
+            step(loop, c + 2, lds2, wv[2], lds3, wv[3]);
+            step(loop, c + 3, lds3, wv[3], lds0, wv[0]);
         }
-        if (c < nch) step(c, lds0, wv[0], lds1, wv[1]);
-        if (c + 1 < nch) step(c + 1, lds1, wv[1], lds2, wv[2]);
-        if (c + 2 < nch) step(c + 2, lds2, wv[2], lds3, wv[3]);
+        if (c < nch) step(tail0, c, lds0, wv[0], lds1, wv[1]);
+        if (c + 1 < nch) step(std::integral_constant<int, 1>{}, c + 1, lds1, wv[1], lds2, wv[2]);
+        if (c + 2 < nch) step(std::integral_constant<int, 2>{}, c + 2, lds2, wv[2], lds3, wv[3]);
     }
     // (no copy into this workgroup's LDS outlives it)
     __builtin_amdgcn_s_waitcnt(0);
