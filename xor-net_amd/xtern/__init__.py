@@ -302,8 +302,13 @@ def _dev_ptr(t, dtype, what):
 
 
 def _rows(x):
-    """x as [rows, columns]."""
-    return x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
+    """x as [rows, columns], and both counts; rows of no columns are reshape's
+    error."""
+    s = x.shape
+    if len(s) != 2 or not s[1]:
+        x = x.reshape(-1, s[-1])
+        s = x.shape
+    return x, s[0], s[1]
 
 
 class DeviceWeights:
@@ -563,8 +568,7 @@ def quantize_i8(x, mode=XT_QUANT_AVX512, stream=None):
     """Device quantize_f32_to_i8 over the rows of x [M, K] (or [K]).
     Returns (q int8 [M, K], inv_scale f32 [M])."""
     torch = _torch()
-    x2 = _rows(x)
-    M, K = x2.shape
+    x2, M, K = _rows(x)
     q = torch.empty((M, K), dtype=torch.int8, device=x.device)
     inv = torch.empty((M,), dtype=torch.float32, device=x.device)
     _check(_lib.xt_quantize_i8(_dev_ptr(x2, torch.float32, "x"), M, K,
@@ -576,8 +580,7 @@ def quantize_i8(x, mode=XT_QUANT_AVX512, stream=None):
 def quantize_i8_rowsum(x, mode=XT_QUANT_AVX512, stream=None):
     """quantize_i8 plus the exact i32 row sums of q (an xtern extension)."""
     torch = _torch()
-    x2 = _rows(x)
-    M, K = x2.shape
+    x2, M, K = _rows(x)
     q = torch.empty((M, K), dtype=torch.int8, device=x.device)
     inv = torch.empty((M,), dtype=torch.float32, device=x.device)
     rs = torch.empty((M,), dtype=torch.int32, device=x.device)
@@ -592,8 +595,7 @@ def quantize_i8_rowsum(x, mode=XT_QUANT_AVX512, stream=None):
 def linear_q_rowsum(w, q, inv, rowsum, out=None, stream=None):
     """linear_q with caller-provided row sums of q (an xtern extension)."""
     torch = _torch()
-    q2 = _rows(q)
-    M = q2.shape[0]
+    q2, M, _ = _rows(q)
     y = out if out is not None else torch.empty((M, w.out_dim), dtype=torch.float32, device=q.device)
     _check(_lib.xt_ternary_linear_q_rowsum(w.handle, _dev_ptr(q2, torch.int8, "q"),
                                            _dev_ptr(inv, torch.float32, "inv_scale"),
@@ -606,11 +608,10 @@ def linear_q_rowsum(w, q, inv, rowsum, out=None, stream=None):
 def linear_q(w, q, inv, acc=False, out=None, stream=None):
     """y = dot(q, W) * inv * w_scales for q [M, K] int8, inv [M] f32."""
     torch = _torch()
-    q2 = _rows(q)
-    M = q2.shape[0]
-    if q2.shape[1] != w.in_dim:
+    q2, M, K = _rows(q)
+    if K != w.in_dim:
         raise XternError(XT_ERR_INVALID,
-                         f"Input dimension mismatch: expected {w.in_dim}, got {q2.shape[1]}")
+                         f"Input dimension mismatch: expected {w.in_dim}, got {K}")
     y = out if out is not None else torch.empty((M, w.out_dim), dtype=torch.float32, device=q.device)
     a = torch.empty((M, w.out_dim), dtype=torch.int32, device=q.device) if acc else None
     _check(_lib.xt_ternary_linear_q(w.handle, _dev_ptr(q2, torch.int8, "q"),
@@ -625,8 +626,7 @@ def linear_f32_noalloc(w, x, mode=XT_QUANT_AVX512, out=None, stream=None):
     """linear_f32 through xt_ternary_linear_f32_noalloc (static device scratch,
     no allocation in the library; calls overlapping on one GPU race)."""
     torch = _torch()
-    x2 = _rows(x)
-    M = x2.shape[0]
+    x2, M, _ = _rows(x)
     y = out if out is not None else torch.empty((M, w.out_dim), dtype=torch.float32, device=x.device)
     _check(_lib.xt_ternary_linear_f32_noalloc(w.handle, _dev_ptr(x2, torch.float32, "x"), M,
                                               _dev_ptr(y, torch.float32, "y"), mode,
@@ -643,8 +643,7 @@ def linear_f32(w, x, mode=XT_QUANT_AVX512, out=None, stream=None):
     """Quantise rows of x [M, K] f32 and apply the ternary product."""
     torch = _torch()
     f32 = torch.float32
-    x2 = _rows(x)
-    M, K = x2.shape
+    x2, M, K = _rows(x)
     if K != w.in_dim:
         raise XternError(XT_ERR_INVALID,
                          f"Input dimension mismatch: expected {w.in_dim}, got {K}")
@@ -675,7 +674,7 @@ def rms_norm(x, weight, eps, out=None, stream=None):
     if weight.numel() != n:
         raise XternError(XT_ERR_INVALID,
                          f"FastTensor::rmsnorm weight size mismatch: expected {n}, got {weight.numel()}")
-    x2 = _rows(x).contiguous()
+    x2 = _rows(x)[0].contiguous()
     y = out if out is not None else torch.empty_like(x2)
     _check(_lib.xt_rms_norm(_dev_ptr(x2, torch.float32, "x"),
                             _dev_ptr(weight.contiguous(), torch.float32, "weight"), x2.shape[0], n,
@@ -694,7 +693,7 @@ def mlp_q(gate, up, down, q, inv, norm_w=None, eps=1e-5, use_silu=False,
     """xt_ternary_mlp_q: fused_mlp_all on every row of q [M, in_dim] i8."""
     torch = _torch()
     _mlp_check(gate, up, down, q.shape[-1])
-    q2 = _rows(q).contiguous()
+    q2 = _rows(q)[0].contiguous()
     M = q2.shape[0]
     y = out if out is not None else torch.empty((M, down.out_dim), dtype=torch.float32,
                                                 device=q.device)
@@ -712,7 +711,7 @@ def mlp_f32(gate, up, down, x, norm_w=None, eps=1e-5, use_silu=False, mode=XT_QU
     """xt_ternary_mlp_f32: Mlp::forward for x [M, in_dim] f32."""
     torch = _torch()
     _mlp_check(gate, up, down, x.shape[-1])
-    x2 = _rows(x).contiguous()
+    x2 = _rows(x)[0].contiguous()
     M = x2.shape[0]
     y = out if out is not None else torch.empty((M, down.out_dim), dtype=torch.float32,
                                                 device=x.device)
@@ -733,8 +732,7 @@ def _multi(ws, ys):
 
 def linear_multi_f32(ws, x, mode=XT_QUANT_AVX512, stream=None, outs=None):
     torch = _torch()
-    x2 = _rows(x)
-    M = x2.shape[0]
+    x2, M, _ = _rows(x)
     ys = outs if outs is not None else [torch.empty((M, w.out_dim), dtype=torch.float32,
                                                     device=x.device) for w in ws]
     harr, yarr = _multi(ws, ys)
@@ -745,8 +743,7 @@ def linear_multi_f32(ws, x, mode=XT_QUANT_AVX512, stream=None, outs=None):
 
 def linear_multi_q(ws, q, inv, stream=None):
     torch = _torch()
-    q2 = _rows(q)
-    M = q2.shape[0]
+    q2, M, _ = _rows(q)
     ys = [torch.empty((M, w.out_dim), dtype=torch.float32, device=q.device) for w in ws]
     harr, yarr = _multi(ws, ys)
     _check(_lib.xt_ternary_linear_multi_q(harr, len(ws), _dev_ptr(q2, torch.int8, "q"),
