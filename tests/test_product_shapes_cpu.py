@@ -46,3 +46,21 @@ def test_narrow_pack5_of_a_million_rows():
     assert choose(xtern.XT_PACK5, BLOCKS * 16, 2, 8).kind == 0  # (as priced, one block inside the limit)
     assert choose(xtern.XT_PACK5, BLOCKS * 16 + 1, 2, 8).kind == 4
     assert choose(xtern.XT_PACK5, 2097120, 6, 1).kind == 4
+
+
+@pytest.mark.parametrize("cfg", ["gw,3,1,4", "gw,4,1,8", "gw,0,0,0", "gw,1,1,-4"])
+def test_a_forced_shape_is_taken_or_refused(cfg, monkeypatch):
+    """A forced shape of the many-row GEMM that is not compiled for the format
+    must not run as another kernel (kind -1: the call fails)."""
+    monkeypatch.setenv("XTERN_CONFIG", cfg)
+    assert choose(xtern.XT_PACK4, 64, 432, 10).kind == -1
+    assert choose(xtern.XT_PACK4, 16, 432, 10).kind == 2  # (no shape of that GEMM below 17 rows)
+
+
+def test_a_forced_shape_keeps_the_offset_limit(monkeypatch):
+    """4 GiB of weight tiles: beyond the kernel's 32-bit offsets."""
+    monkeypatch.setenv("XTERN_CONFIG", "gw,4,2,4")
+    c = choose(xtern.XT_PACK4, 64, 65535, 64)
+    assert (c.kind, c.mb, c.nb, c.waves) == (4, 8, 16, 4)
+    assert choose(xtern.XT_PACK4, 64, 65536, 64).kind == -1
+    assert choose(xtern.XT_PACK4, 64, 16, 1 << 16).kind == -1

@@ -290,6 +290,7 @@ int run_product(const xt_weights* const* ws, int n, const int8_t* q, int ldq, co
     }
     const xt::MMConfig cfg =
         xt::choose_config(fmt, (int)M, ng_total, (int)ws[0]->nch, rowsum != nullptr);
+    if (cfg.kind < 0) return fail(XT_ERR_UNSUPPORTED, "XTERN_CONFIG names no shape that takes this product");
     xt::MMArgs a;
     memset(&a, 0, sizeof a);
     int tiles = 0, cols = 0;

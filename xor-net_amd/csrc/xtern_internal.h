@@ -93,7 +93,8 @@ struct MMConfig {
     int mb, nb, waves, pf;  // tokens per WG = 16*mb, rows per WG = 16*nb
     int splitk;             // workgroups along K (blockIdx.z)
     int kind = 0;           // 0 mm_kernel, 2 decode GEMV (waves used), 4 gemmw_kernel
-                            // (mb = 2 mw, nb = 2 nw waves)
+                            // (mb = 2 mw, nb = 2 nw waves), -1 a forced shape that
+                            // cannot take the product
 };
 
 // Kernel launchers (xtern_kernels.hip).  Return the hipError_t of the launch.

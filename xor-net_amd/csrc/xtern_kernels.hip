@@ -1427,9 +1427,13 @@ const GemmShape kShapes5[] = {
     {8, 8, 4, 1, 4, 1.300f, 1.300f, 3.0f, 1}, {8, 16, 8, 1, 4, 2.000f, 2.200f, 3.5f, 1},
 };
 
+// gemmw_kernel's byte offsets within a matrix and a token block are 32-bit.
+bool gemmw_offsets(int ngroups, int nch) {
+    return (size_t)ngroups * nch * kTileBytes < ((size_t)1 << 32) && nch < (1 << 16);
+}
+
 MMConfig choose_gemm(int fmt, int M, int ngroups, int nch) {
-    // gemmw_kernel's byte offsets within a matrix and a token block are 32-bit
-    const bool wide = (size_t)ngroups * nch * kTileBytes < ((size_t)1 << 32) && nch < (1 << 16);
+    const bool wide = gemmw_offsets(ngroups, nch);
     MMConfig best;
     double best_cost = -1.0;
     auto take = [&](const GemmShape& g) {
@@ -1460,7 +1464,13 @@ MMConfig choose_config(int fmt, int M, int ntiles_nb1, int nch, bool have_rowsum
             c.nb = gemv_row_groups(fmt, nch, ntiles_nb1);
             return c;
         }
-        if (c.kind == 4 && M > 16 && gemmw_known(fmt, c.mb / 2, c.nb / (2 * c.waves), c.waves)) return c;
+        // (a forced shape of the many-row GEMM is taken or refused: kind -1)
+        if (c.kind == 4 && M > 16) {
+            if (!gemmw_known(fmt, c.mb / 2, c.waves > 0 ? c.nb / (2 * c.waves) : 0, c.waves) ||
+                !gemmw_offsets(ntiles_nb1, nch))
+                c.kind = -1;
+            return c;
+        }
         if (c.kind == 0 && shape_known(c, !have_rowsum)) {
             if (c.splitk > nch) c.splitk = nch;
             return c;
