@@ -1325,7 +1325,8 @@ hipError_t launch_gemv(int fmt, const MMArgs& a, int ntiles, int waves, hipStrea
     return hipErrorInvalidValue;
 }
 
-// Compiled tile shapes, selectable by MMConfig.
+// Compiled tile shapes, selectable by MMConfig; (1, 1, 4, 4), (1, 4, 4, 2) and
+// (2, 8, 4, 2) run only when forced, and carry the tests of split K.
 #define XT_MM_SHAPES(X)  \
     X(1, 1, 4, 4)        \
     X(1, 1, 8, 2)        \
@@ -1346,16 +1347,12 @@ bool shape_known(const MMConfig& c, bool own) {
     return false;
 }
 
-// XTERN_CONFIG="mb,nb,waves,pf,splitk" forces one tile shape (for tuning),
-// "g32,S" S slices of K over workgroups, "gw,mw,nw,waves" one shape of the
-// many-row GEMM, "gemv,W" the decode GEMV.
+// XTERN_CONFIG="mb,nb,waves,pf,splitk" forces one tile shape (for tuning; the
+// only way to splitk > 1 slices of K over workgroups), "gw,mw,nw,waves" one
+// shape of the many-row GEMM, "gemv,W" the decode GEMV.
 bool env_config(MMConfig* c) {
     const char* e = getenv("XTERN_CONFIG");
     MMConfig f;
-    if (e && sscanf(e, "g32,%d", &f.splitk) == 1 && f.splitk >= 1) {
-        *c = MMConfig{1, 4, 4, 2, f.splitk};
-        return true;
-    }
     int mw = 0, nw = 0, w = 0;
     if (e && sscanf(e, "gw,%d,%d,%d", &mw, &nw, &w) == 3) {
         f = MMConfig{2 * mw, 2 * nw * w, w, 1, 1};
