@@ -61,6 +61,26 @@ def test_fused_row_exact(fmt, mode):
             assert np.array_equal(y.view(np.int32), ref.view(np.int32)), f"{int(np.sum(y != ref))} differ"
 
 
+@pytest.mark.parametrize("fmt,K,N", [(xtern.XT_PACK4, 8196, 40), (xtern.XT_XORSPARSE, 8448, 640),
+                                     (xtern.XT_PACK4, 9020, 100), (xtern.XT_PACK4, 9216, 320),
+                                     (xtern.XT_XORSPARSE, 9216, 17), (xtern.XT_PACK4, 9220, 40),
+                                     (xtern.XT_PACK5, 8964, 40)])
+def test_longest_fused_rows_exact(fmt, K, N):
+    """Rows around the longest that the GEMV quantises (36 chunks of 256, three
+    per wave of the last instantiation; Pack5 28 of 320): 9220 and 8964 take
+    the separate quantiser."""
+    rng = np.random.default_rng(K)
+    print(f"[case] longest fused row fmt={fmt} K={K} N={N}", flush=True)
+    ws = rng.uniform(0.2, 2.0, N).astype(np.float32)
+    t, w = weights(rng, fmt, K, N, ws)
+    for m in (xtern.XT_QUANT_AVX512, xtern.XT_QUANT_SCALAR):
+        for x in rows(rng, K):
+            q, inv = oracle.quantize(x, m)
+            y = xtern.linear_f32(w, torch.from_numpy(x[None]).to(DEV), mode=m).cpu().numpy()
+            ref = product(t, np.asarray(q).reshape(1, K), np.float32(inv).reshape(1), ws)
+            assert np.array_equal(y.view(np.int32), ref.view(np.int32)), f"{int(np.sum(y != ref))} differ"
+
+
 @pytest.mark.parametrize("K,N", [(512, 80), (1000, 777), (4096, 640)])
 def test_stream_row_counts(K, N):
     rng = np.random.default_rng(K + N)

@@ -404,7 +404,7 @@ int gemv_fused_quant(const xt_weights* const* ws, int n, const float* x, int64_t
     // few us against the ~50 us of a 128256-row head (measured: Int8 head
     // forward 158 us fused on the staged GEMV, 50 us product on this one)
     if (xt::is_int_format(fmt) && xt::gemv2_takes(fmt, nch)) return 1;
-    if (M > 16 || M * K > (direct ? xt::kGemv2FusedQuantMax : xt::kGemvFusedQuantMax) ||
+    if (M > 16 || (!direct && M * K > xt::kGemvFusedQuantMax) ||
         (((uintptr_t)x) & 15) || (K & 3))
         return 1;
     int ng_total = 0;
@@ -424,11 +424,11 @@ int gemv_fused_quant(const xt_weights* const* ws, int n, const float* x, int64_t
         const int g = xt::gemv_row_groups(fmt, nch, ng_total);
         if ((int64_t)((ng_total + g - 1) / g) * K > kFusedRowReads) return 1;
     }
-    // Ternary tiles take the staging-free GEMV (one chunk per wave, so
-    // K <= 16 chunks); Int8 / Int4 the staged one (one piece per thread).
+    // Ternary tiles take the staging-free GEMV, Int8 / Int4 the staged one
+    // (one piece per thread).
     const int segs = xt::chunk_cols(fmt) / 16;
     const int rg = direct ? xt::gemv_row_groups(fmt, nch, ng_total) : 1;
-    if (direct ? (M * K > xt::gemv2_fused_max(fmt, nch, rg))
+    if (direct ? !xt::gemv2_fuses(fmt, nch)
                : (!xt::gemv_fits(fmt, (int)M, nch, waves, xt::gemv_ncw(waves)) ||
                   M * nch * segs > (int64_t)waves * 64))
         return 1;

@@ -65,12 +65,10 @@ struct MMArgs {
     int rg;                 // decode GEMV: 16-row groups per workgroup (0 or 1: one)
     int gx;                 // gemmw_kernel: workgroup columns (set by its launcher)
 };
-// GEMV with the quantiser fused when M * K is at most this (every workgroup
-// re-reads the f32 rows, so only for small inputs).  The staging-free GEMV
-// fuses one row of up to this many columns (its LDS stage bounds K further:
-// 31 Pack4 or 28 Pack5 chunks).
+// The staged GEMV (Int8 / Int4 rows, or K beyond the staging-free one) with the
+// quantiser fused when M * K is at most this: every workgroup re-reads the f32
+// rows, so only for small inputs.
 constexpr int kGemvFusedQuantMax = 8192;
-constexpr int kGemv2FusedQuantMax = 16384;
 
 // Streaming decode GEMV (xtern_gstream.hip): one projection, M <= 16 rows
 // of i8 activations given.
@@ -113,9 +111,8 @@ hipError_t launch_gemmw(int fmt, int mw, int nw, int w, const MMArgs& a, int nti
 // Decode GEMV (M <= 16): 16 output rows per workgroup, activations in LDS.
 hipError_t launch_gemv(int fmt, const MMArgs& a, int ntiles, int waves, hipStream_t s);
 int gemv_ncw(int waves);
-// Largest M * K the staging-free GEMV quantises itself for nch chunks and rg
-// row groups per workgroup (0: none).
-int gemv2_fused_max(int fmt, int nch, int rg);
+// Whether the staging-free GEMV takes one f32 row of nch chunks.
+bool gemv2_fuses(int fmt, int nch);
 // 16-row groups per workgroup of the decode GEMV that launch_gemv runs for
 // this format and K (its ntiles count workgroups of that many groups).
 int gemv_row_groups(int fmt, int nch, int ngroups);

@@ -1159,24 +1159,15 @@ static int gemv2_rg_for(int fmt, int nch, int ngroups) {
     return 1;
 }
 
-// Waves of the staging-free GEMV for nch chunks.
-static int gemv2_waves(int nch) {
-    for (int w : {4, 8, 10, 16})
-        if (nch <= w) return w;
-    // (as the launcher's list: 14 waves where they cover K at 2, 3 or 4
-    // chunks per wave)
-    return (nch <= 28 || (nch > 32 && nch <= 42) || (nch > 48 && nch <= 56)) ? 14 : 16;
-}
-// Longest f32 row the fused GEMV takes: rows of at most about 36 (Pack5 28)
-// chunks, so that the row's registers and the workgroups' repeated reads of
-// it stay small; longer rows take the quantiser launch.  (Every workgroup
-// quantises the whole row: 4096 -> 14336, 448 workgroups, 10.1 us fused vs
-// 8.6 with the launch.)
-int gemv2_fused_max(int fmt, int nch, int rg) {
-    const int steps = fmt == XT_PACK5 ? 5 : 4, w = gemv2_waves(nch);
-    if (nch > 64 || nch * steps * 1024 + w * rg * 64 * 16 + w * 16 * 4 > 160 * 1024) return 0;
-    return w * 64 * 32;
-}
+// Chunks of the longest f32 row that the GEMV quantises itself; longer rows
+// take the quantiser launch.  Below the line the fused form saves that launch
+// (launch to launch, us, fused / with the launch, to 640 outputs: Pack4 4096
+// 3.4 / 5.3, 9216 5.7 / 7.4; Pack5 8960 6.9 / 7.8).  The line is no optimum:
+// it lies where the LDS stage of an earlier form that took several rows ended,
+// and the one-row form would gain beyond it as well (Pack4 9472 5.9 / 7.5,
+// 16384 7.3 / 8.9; Pack5 9280 7.0 / 7.8).
+constexpr int fused_chunks(int fmt) { return fmt == XT_PACK5 ? 28 : 36; }
+bool gemv2_fuses(int fmt, int nch) { return nch <= fused_chunks(fmt); }
 
 // Quantised rows given: the activation pieces through a wave-private LDS
 // slice when the wave multiplies two or more chunks and the slice of M rows
@@ -1239,18 +1230,29 @@ static hipError_t launch_gemv2_int(const MMArgs& a, int ntiles, hipStream_t s) {
     return hipGetLastError();
 }
 
+// One f32 row quantised in the kernel: compiled for the waves and chunks per
+// wave that rows of up to fused_chunks(FMT) reach (14 x 2 for Pack5, 14 x 3
+// for Pack4).
+template <int FMT, int W, int NCW, int RG>
+static hipError_t launch_gemv2_fused(const MMArgs& a, int ntiles, hipStream_t s) {
+    if constexpr (W * NCW <= (fused_chunks(FMT) + 13) / 14 * 14) {
+        hipLaunchKernelGGL((gemv2_kernel<FMT, W, NCW, true, RG>), dim3(ntiles), dim3(W * 64), 0, s, a);
+        return hipGetLastError();
+    }
+    return hipErrorInvalidValue;
+}
+
 // The staging-free GEMV applies to ternary tiles (given or fused-quantised rows).
 template <int RG>
 static hipError_t launch_gemv2_rg(int fmt, const MMArgs& a, int ntiles, hipStream_t s) {
     const int nch = a.nch;
-    if (a.x && (a.M != 1 || a.K > gemv2_fused_max(fmt, nch, RG))) return hipErrorInvalidValue;
+    if (a.x && (a.M != 1 || !gemv2_fuses(fmt, nch))) return hipErrorInvalidValue;
 #define XT_GV2(W_, NCW_)                                                                         \
     if (nch <= W_ * NCW_) {                                                                      \
         if (a.x) {                                                                               \
             if (fmt == XT_PACK5)                                                                 \
-                hipLaunchKernelGGL((gemv2_kernel<XT_PACK5, W_, NCW_, true, RG>), dim3(ntiles), dim3(W_ * 64), 0, s, a);\
-            else                                                                                 \
-                hipLaunchKernelGGL((gemv2_kernel<XT_PACK4, W_, NCW_, true, RG>), dim3(ntiles), dim3(W_ * 64), 0, s, a);\
+                return launch_gemv2_fused<XT_PACK5, W_, NCW_, RG>(a, ntiles, s);                 \
+            return launch_gemv2_fused<XT_PACK4, W_, NCW_, RG>(a, ntiles, s);                     \
         } else if (fmt == XT_PACK5) {                                                            \
             return launch_gemv2_am<XT_PACK5, W_, NCW_, RG>(a, ntiles, s);                      \
         } else if (fmt == XT_INT8) {                                                             \
@@ -1266,7 +1268,6 @@ static hipError_t launch_gemv2_rg(int fmt, const MMArgs& a, int ntiles, hipStrea
         } else {                                                                                 \
             return launch_gemv2_am<XT_PACK4, W_, NCW_, RG>(a, ntiles, s);                      \
         }                                                                                        \
-        return hipGetLastError();                                                                \
     }
     // Pack5 at 5..10 chunks: five waves of two chunks (measured, 3200 ->
     // 8640: 4.8 vs 5.3 us at M = 1, 6.0 vs 6.2 at M = 8; Pack4 is fastest
