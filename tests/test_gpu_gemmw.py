@@ -57,6 +57,24 @@ def test_forced_shapes_exact(fmt, shape, monkeypatch):
         assert bool((guard[M] == 7.0).all())
 
 
+@pytest.mark.parametrize("fmt,shape", [(xtern.XT_PACK4, s) for s in PACK4] + [(xtern.XT_PACK5, s) for s in PACK5])
+def test_forced_shapes_several_projections(fmt, shape, monkeypatch):
+    """Projections of one launch that end inside a tile of every shape, the first
+    or second wide enough that a later one starts past several tiles."""
+    monkeypatch.setenv("XTERN_CONFIG", "gw," + shape)
+    rng = np.random.default_rng(12)
+    ch = 320 if fmt == xtern.XT_PACK5 else 256
+    for M, K, widths in ((33, 2 * ch, (700, 96, 33)), (150, 3 * ch, (33, 700, 96, 1)), (17, ch, (256, 257))):
+        print(f"[case] gw,{shape} fmt={fmt} M={M} K={K} N={widths}", flush=True)
+        q = rng.integers(-128, 128, (M, K)).astype(np.int8)
+        inv = rng.uniform(1e-3, 0.1, M).astype(np.float32)
+        scales = [rng.uniform(0.2, 2.0, N).astype(np.float32) for N in widths]
+        made = [weights(rng, fmt, K, N, s) for N, s in zip(widths, scales)]
+        ys = xtern.linear_multi_q([w for _, w in made], torch.from_numpy(q).to(DEV), torch.from_numpy(inv).to(DEV))
+        for (t, _), s, y in zip(made, scales, ys):
+            assert np.array_equal(y.cpu().numpy().view(np.int32), reference(t, q, inv, s)[1])
+
+
 @pytest.mark.parametrize("fmt", [xtern.XT_PACK4, xtern.XT_PACK5], ids=["pack4", "pack5"])
 @pytest.mark.parametrize("M", [17, 64, 200, 600])
 def test_chosen_shapes_match_single_projections(fmt, M):

@@ -60,28 +60,33 @@ def test_activation_widths(M, n):
     r = np.maximum(g, np.float32(0))
     assert np.array_equal(bits(got), bits((r * r).astype(np.float32) * u))
     wide = xtern.activation_mul(xtern.XT_ACT_SILU_INPLACE_SCALAR, gd, ud)
-    for m in (0, M - 1):  # (a row alone takes another width)
+    for m in (0, M // 2, M - 1):  # (a row alone can take another width)
         one = xtern.activation_mul(xtern.XT_ACT_SILU_INPLACE_SCALAR, gd[m:m + 1], ud[m:m + 1])
         assert torch.equal(one[0].view(torch.int32), wide[m].view(torch.int32))
+        ref = oracle.silu_inplace(g[m], u[m], True, avx512=False)
+        assert np.array_equal(bits(wide[m].cpu().numpy()), bits(ref))
 
 
 @pytest.mark.parametrize("norm", [False, True])
 @pytest.mark.parametrize("M,K,I", [(2, 64, 1024), (300, 64, 1020), (520, 64, 4608), (3, 64, 4613)])
 def test_mlp_rows_match_single_row(M, K, I, norm):
     """The MLP of many rows equals each row's (ReLU^2: one row takes the same
-    function), through the requantisation of every width."""
+    function) and the oracle's, through the requantisation of every width."""
     print(f"[case] mlp M={M} K={K} I={I} norm={norm}", flush=True)
     rng = np.random.default_rng(I + M)
 
     def lin(k, n):
         t = rng.integers(-1, 2, (n, k)).astype(np.int8)
-        return xtern.DeviceWeights(xtern.XT_PACK4, k, n, np.concatenate([xtern.pack_ternary4(r) for r in t]),
-                                   np.full(n, 0.7, np.float32))
+        b, ws = np.concatenate([xtern.pack_ternary4(r) for r in t]), np.full(n, 0.7, np.float32)
+        return xtern.DeviceWeights(xtern.XT_PACK4, k, n, b, ws), (xtern.XT_PACK4, k, n, ws, dict(wbytes=b))
 
-    gate, up, down = lin(K, I), lin(K, I), lin(I, 48)
+    (gate, go), (up, uo), (down, do) = lin(K, I), lin(K, I), lin(I, 48)
     w = torch.rand(I, device=DEV) + 0.5 if norm else None
     x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32)).to(DEV)
     y = xtern.mlp_f32(gate, up, down, x, norm_w=w)
     for m in (0, M // 2, M - 1):
         one = xtern.mlp_f32(gate, up, down, x[m:m + 1], norm_w=w)
         assert torch.equal(one[0].view(torch.int32), y[m].view(torch.int32))
+        ref = oracle.mlp_forward(x[m:m + 1].cpu().numpy(), go, uo, do, w.cpu().numpy() if norm else None, 1e-5,
+                                 False, fused=False)[0]
+        assert np.array_equal(bits(y[m].cpu().numpy()), bits(ref[0]))

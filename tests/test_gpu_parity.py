@@ -431,6 +431,23 @@ def test_forced_splitk_configs(cfg, monkeypatch):
         assert np.array_equal(acc.cpu().numpy(), exact_acc(t, q))
 
 
+@pytest.mark.parametrize("cfg", ["2,8,4,2,4", "2,8,4,2,1", "1,4,4,2,3"])
+def test_forced_configs_with_row_sums(cfg, monkeypatch):
+    """Row sums given by the caller: the only calls that a forced shape of 32
+    tokens takes."""
+    monkeypatch.setenv("XTERN_CONFIG", cfg)
+    rng = np.random.default_rng(41)
+    for K, N, M in ((2560, 640, 1), (6912, 2560, 128), (2560, 6912, 40), (1024, 96, 16)):
+        log(f"forced with row sums {cfg} K={K} N={N} M={M}")
+        t = tern(rng, N, K)
+        w = xtern.DeviceWeights(xtern.XT_PACK4, K, N, make_bytes(t, xtern.XT_PACK4),
+                                np.ones(N, np.float32))
+        q = rng.integers(-127, 128, (M, K)).astype(np.int8)
+        y = xtern.linear_q_rowsum(w, torch.from_numpy(q).to(DEV), torch.ones(M, device=DEV),
+                                  torch.from_numpy(q.astype(np.int32).sum(1, dtype=np.int32)).to(DEV))
+        assert np.array_equal(y.cpu().numpy(), exact_acc(t, q).astype(np.float32))
+
+
 @pytest.mark.parametrize("mode", [xtern.XT_QUANT_AVX512, xtern.XT_QUANT_SCALAR])
 @pytest.mark.parametrize("fmt", FMTS)
 @pytest.mark.parametrize("M,K", [(1, 4), (1, 16), (1, 20), (2, 100), (3, 2560), (1, 8192),
