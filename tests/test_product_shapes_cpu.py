@@ -64,3 +64,22 @@ def test_a_forced_shape_keeps_the_offset_limit(monkeypatch):
     assert (c.kind, c.mb, c.nb, c.waves) == (4, 8, 16, 4)
     assert choose(xtern.XT_PACK4, 64, 65536, 64).kind == -1
     assert choose(xtern.XT_PACK4, 64, 16, 1 << 16).kind == -1
+
+
+@pytest.mark.parametrize("M,K,N,mb,nb", [
+    # one workgroup per CU at most: the smallest tile starts first (16 x 32
+    # against 16 x 64, us: 5.3 / 5.8, 4.1 / 4.6, 5.0 / 6.2)
+    (17, 4096, 2560, 1, 2), (17, 2048, 1024, 1, 2), (128, 4096, 640, 1, 2),
+    # 25 columns of 16 x 128 tiles over 8 XCDs: each reads all of the weights
+    # (against 32 x 128: 10.9 / 8.2, 9.2 / 6.9, 7.0 / 5.6)
+    (128, 4096, 3200, 2, 8), (160, 3072, 3200, 2, 8), (64, 2048, 6912, 2, 8),
+    # columns that divide over the XCDs (8.6 / 10.0)
+    (128, 5120, 4096, 1, 8),
+    # large activations, read again by every column (15.4 / 13.3)
+    (512, 14336, 256, 1, 4),
+])
+def test_pack4_shapes_measured_fastest(M, K, N, mb, nb, monkeypatch):
+    monkeypatch.delenv("XTERN_CONFIG", raising=False)
+    for fmt in (xtern.XT_PACK4, xtern.XT_XORSPARSE):
+        c = choose(fmt, M, -(-N // 16), -(-K // 256))
+        assert (c.mb, c.nb) == (mb, nb)

@@ -11,6 +11,7 @@
 #include <stdio.h>
 #include <stdlib.h>
 
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -1387,31 +1388,44 @@ int int_gemv_waves(int fmt, int mb, int nch) {
 }
 
 namespace {
-// Shapes of a product with more than 16 rows, and what one workgroup of each
-// costs per chunk of K: `first` when it has its CU to itself, `rest` for each
-// further workgroup of the CU, `gap` once per further workgroup (its start and
-// epilogue, as far as they are not hidden; microseconds; `unit`: K is taken
-// in rounds of so many chunks).  Fitted to launch-to-launch
-// times on MI355X over M = 20 .. 2048 and K, N = 512 .. 14336 (weights
-// streamed from memory); with a few launches more or less per CU the totals
-// are within about 15 % of the measured ones, and where two shapes come out
-// close they measure close.
+// Shapes of a product with more than 16 rows, and what one of them costs in
+// microseconds: `start` once; per chunk of K (K in rounds of `unit` chunks)
+// `first` for a workgroup that has its CU to itself, `rest` for each further
+// one of the busiest CU, and `gap` once per further one (its start and
+// epilogue, as far as they are not hidden).  `spread`: mm_kernel's workgroup t
+// runs on XCD t % 8, so a column of weights that more than one XCD multiplies
+// is read into the L2 of each; per chunk, with all 8 of them and every CU
+// taken.  `acts`: most KiB of activations (0: any).
+// Pack4: fitted to launch-to-launch times on MI355X of all eight shapes at
+// 2047 sizes (M = 17 .. 4096, K = 256 .. 14336, N = 100 .. 17280, weights
+// streamed from memory): the shape chosen is 0.8 % slower than the fastest on
+// average and within 3 % of it at nine sizes of ten.
 struct GemmShape {
     int mb, nb, waves, pf, kind;
-    float first, rest, gap;
-    int unit;
+    float start, first, spread, rest, gap;
+    int unit, acts;
 };
-// 16-token shapes (mm_kernel) win while every CU gets at most one of them;
-// then ever larger tiles of gemmw_kernel.  Examples, us (16 x 64 / 16 x 128 /
-// 32 x 128 / 64 x 128 / 64 x 256 / 128 x 256): 2560 -> 6912 at M = 32 6.2 /
-// 7.4 / 6.7 / 9.4 / 13 / 20, at M = 512 - / - / 16.5 / 14.2 / 14.0 / 20.4, at
-// M = 2048 - / - / 47 / 41 / 39 / 38; 6912 -> 2560 at M = 64 7.9 / 10.7 /
-// 11.9 / 13.9 / 22 / 42, at M = 512 - / - / 18.7 / 15.9 / 24 / 39.
+// 16-token shapes (mm_kernel) win while every CU gets at most one of them, 32
+// output rows before 64 and more (the smallest start; us, 16 x 32 / 16 x 64 /
+// 32 x 128: 4096 -> 2560 at M = 17 5.3 / 5.8 / 8.3, 4096 -> 640 at M = 128
+// 5.0 / 6.2 / 7.9), except that its many columns read large activations again
+// and again (14336 -> 256 at M = 512: 15.4 / 13.3); 16 x 128 where its columns
+// divide over the XCDs (/ 32 x 128: 5120 -> 4096 at M = 128 8.6 / 10.0, but
+// 4096 -> 3200 10.9 / 8.2); then ever larger tiles of gemmw_kernel.  Examples,
+// us (16 x 64 / 16 x 128 / 32 x 128 / 64 x 128 / 64 x 256 / 128 x 256): 2560
+// -> 6912 at M = 32 6.2 / 7.4 / 6.7 / 9.4 / 13 / 20, at M = 512 - / - / 16.5 /
+// 14.2 / 14.0 / 20.4, at M = 2048 - / - / 47 / 41 / 39 / 38; 6912 -> 2560 at
+// M = 64 7.9 / 10.7 / 11.9 / 13.9 / 22 / 42, at M = 512 - / - / 18.7 / 15.9 /
+// 24 / 39.
 const GemmShape kShapes4[] = {
-    {1, 2, 4, 4, 0, 0.170f, 0.170f, 1.0f, 1},  {1, 4, 8, 2, 0, 0.160f, 0.160f, 1.2f, 8},
-    {1, 5, 8, 2, 0, 0.190f, 0.190f, 1.2f, 8},  {1, 8, 8, 2, 0, 0.245f, 0.245f, 1.2f, 8},
-    {2, 8, 4, 1, 4, 0.330f, 0.270f, 0.45f, 1}, {4, 8, 4, 1, 4, 0.480f, 0.450f, 0.6f, 1},
-    {4, 16, 4, 1, 4, 0.850f, 0.830f, 0.7f, 1}, {8, 16, 4, 1, 4, 1.570f, 1.450f, 1.5f, 1},
+    {1, 2, 4, 4, 0, 2.54f, 0.150f, 0.099f, 0.170f, 1.00f, 1, 1750},
+    {1, 4, 8, 2, 0, 2.80f, 0.145f, 0.128f, 0.160f, 1.20f, 1, 0},
+    {1, 5, 8, 2, 0, 3.18f, 0.143f, 0.157f, 0.190f, 1.20f, 1, 0},
+    {1, 8, 8, 2, 0, 3.31f, 0.260f, 0.123f, 0.245f, 1.20f, 1, 0},
+    {2, 8, 4, 1, 4, 2.40f, 0.338f, 0.0f, 0.294f, 0.45f, 1, 0},
+    {4, 8, 4, 1, 4, 3.09f, 0.396f, 0.0f, 0.437f, 0.95f, 1, 0},
+    {4, 16, 4, 1, 4, 3.82f, 0.850f, 0.0f, 0.826f, 0.82f, 1, 0},
+    {8, 16, 4, 1, 4, 4.72f, 1.673f, 0.0f, 1.316f, 1.38f, 1, 0},
 };
 // Pack5 (the base-3 decode is 24 vector instructions per 16 weights against
 // 9, so shapes that decode a weight once for 128 tokens pay earlier): 3200 ->
@@ -1419,10 +1433,14 @@ const GemmShape kShapes4[] = {
 // 15.5 / 12.2 / 16.6 / 22.1, M = 512 32 / 27.8 / 33.7 / 25.6, M = 2048 103 /
 // 77 / 83 / 75.
 const GemmShape kShapes5[] = {
-    {1, 2, 4, 4, 0, 0.290f, 0.160f, 0.0f, 1}, {1, 4, 8, 2, 0, 0.270f, 0.200f, 0.0f, 8},
-    {1, 5, 8, 2, 0, 0.310f, 0.220f, 0.0f, 8}, {1, 5, 16, 1, 0, 0.275f, 0.360f, 0.0f, 16},
-    {2, 8, 4, 1, 4, 0.650f, 0.500f, 0.8f, 1}, {4, 8, 4, 1, 4, 0.800f, 0.620f, 2.2f, 1},
-    {8, 8, 4, 1, 4, 1.300f, 1.300f, 3.0f, 1}, {8, 16, 8, 1, 4, 2.000f, 2.200f, 3.5f, 1},
+    {1, 2, 4, 4, 0, 0.0f, 0.290f, 0.0f, 0.160f, 0.0f, 1, 0},
+    {1, 4, 8, 2, 0, 0.0f, 0.270f, 0.0f, 0.200f, 0.0f, 8, 0},
+    {1, 5, 8, 2, 0, 0.0f, 0.310f, 0.0f, 0.220f, 0.0f, 8, 0},
+    {1, 5, 16, 1, 0, 0.0f, 0.275f, 0.0f, 0.360f, 0.0f, 16, 0},
+    {2, 8, 4, 1, 4, 0.0f, 0.650f, 0.0f, 0.500f, 0.8f, 1, 0},
+    {4, 8, 4, 1, 4, 0.0f, 0.800f, 0.0f, 0.620f, 2.2f, 1, 0},
+    {8, 8, 4, 1, 4, 0.0f, 1.300f, 0.0f, 1.300f, 3.0f, 1, 0},
+    {8, 16, 8, 1, 4, 0.0f, 2.000f, 0.0f, 2.200f, 3.5f, 1, 0},
 };
 
 // gemmw_kernel's byte offsets within a matrix and a token block are 32-bit.
@@ -1436,13 +1454,19 @@ MMConfig choose_gemm(int fmt, int M, int ngroups, int nch) {
     double best_cost = -1.0;
     auto take = [&](const GemmShape& g) {
         const long blocks = (M + 16 * g.mb - 1) / (16 * g.mb);
-        const long tiles = blocks * ((ngroups + g.nb - 1) / g.nb);
+        const long columns = (ngroups + g.nb - 1) / g.nb;
+        const long tiles = blocks * columns;
+        if (g.acts > 0 && (long)M * nch > g.acts * 4L) return;  // (256 bytes a chunk)
         if (g.kind == 4 && (!wide || tiles > 0x7fffffff)) return;
         // (mm_kernel's row blocks are its grid's y; gemmw_kernel's grid has x only)
         if (g.kind == 0 && wide && blocks > 65535) return;
         const long n = (tiles + 255) / 256;  // workgroups of the busiest CU
         const double nc = (nch + g.unit - 1) / g.unit * g.unit;
-        const double cost = g.first * nc + (double)(n - 1) * (g.rest * nc + g.gap);
+        const long period = columns % 8 == 0 ? 1 : columns % 4 == 0 ? 2 : columns % 2 == 0 ? 4 : 8;
+        const double others = (double)(std::min(blocks, period) - 1) / 7.0;  // XCDs that read a column again
+        const double used = (double)std::min(tiles, 256L) / 256.0;
+        const double cost = g.start + nc * (g.first + g.spread * others * used) +
+                            (double)(n - 1) * (g.rest * nc + g.gap);
         if (best_cost >= 0.0 && cost >= best_cost) return;
         best_cost = cost;
         best = MMConfig{g.mb, g.nb, g.waves, g.pf, 1, g.kind};

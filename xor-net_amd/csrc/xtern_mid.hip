@@ -248,7 +248,10 @@ __device__ float seq_advance(float s, const float* lt, int j, int end) {
             acc += min(q + (r == 2 ? 1u : 0u), kGrid);
             pre[k] = acc;  // <= 4 * 2^24 per lane
         }
-        const uint32_t lincl = wave_scan_add(acc);  // <= 256 * 2^24 < 2^32
+        // <= 256 * 2^24 = 2^32.  (Exactly 2^32 wraps to 0 in lane 63 only; then
+        // the lane's exclusive prefix, at most 252 * 2^24, is right, and its
+        // first element is a stop: S + lexcl + pre >= 2^24 in 64 bits.)
+        const uint32_t lincl = wave_scan_add(acc);
         const uint32_t lexcl = lincl - acc;
         // first element (in order) that is a stop or leaves the binade
         int kfirst = kbad;
