@@ -49,7 +49,9 @@ def test_rms_norm_widths(M, n):
 
 
 @pytest.mark.parametrize("M,n", [(3, 1024), (300, 1024), (300, 1023), (3, 1025), (2, 4096), (2, 4100), (3, 8195),
-                                 (515, 8200), (514, 10244), (2, 16384)])
+                                 (515, 8200), (514, 10244), (2, 16384), (5, 1), (3, 17), (300, 64), (4100, 255),
+                                 (3, 256), (3, 257), (512, 512), (513, 512), (513, 511), (2, 513), (256, 1003),
+                                 (257, 1003)])
 def test_activation_widths(M, n):
     print(f"[case] act M={M} n={n}", flush=True)
     rng = np.random.default_rng(n)
@@ -68,7 +70,8 @@ def test_activation_widths(M, n):
 
 
 @pytest.mark.parametrize("norm", [False, True])
-@pytest.mark.parametrize("M,K,I", [(2, 64, 1024), (300, 64, 1020), (520, 64, 4608), (3, 64, 4613)])
+@pytest.mark.parametrize("M,K,I", [(2, 64, 1024), (300, 64, 1020), (520, 64, 4608), (3, 64, 4613), (3, 64, 240),
+                                   (4, 64, 333), (5, 64, 700)])
 def test_mlp_rows_match_single_row(M, K, I, norm):
     """The MLP of many rows equals each row's (ReLU^2: one row takes the same
     function) and the oracle's, through the requantisation of every width."""

@@ -449,10 +449,14 @@ __device__ __forceinline__ float exact_seq_sum(int n, const float* lt, SeqSumLds
     return sl.res;
 }
 
+// How a thread's elements lie in the row: pieces of four (rows of whole,
+// 16-byte aligned pieces), single elements, or one single element in all.
+constexpr int kPieces = 1, kSingles = 0, kOne = 2;
+
 // One workgroup of NT threads per row; thread t holds C4 groups of four
-// elements in registers from the load to the quantisation: VEC (rows of
-// whole, 16-byte aligned pieces) pieces t, t + NT, ..., else elements t,
-// t + NT, ... (so that a wave's loads stay contiguous).  NORM: with RMSNorm.
+// elements (kOne: one element) in registers from the load to the quantisation:
+// pieces t, t + NT, ... or elements t, t + NT, ... (so that a wave's loads stay
+// contiguous).  NORM: with RMSNorm.
 //
 // A row is bound by latency (the load, the walk of the sum, six barriers), so
 // the width is what keeps enough rows in flight: see launch_mlp_mid.
@@ -461,19 +465,22 @@ __device__ __forceinline__ float exact_seq_sum(int n, const float* lt, SeqSumLds
 // 15.8 us, one row of 6912 11.1 -> 8.2, 512 x 6912 22.3 -> 13.8; silu_mul
 // (no norm, f32 out) of 1024 x 8640 34.9 -> 24.6 (4.3 TB/s), the expf in
 // double precision.
-template <int ACT, int NT, int C4, bool VEC, bool NORM>
+template <int ACT, int NT, int C4, int LIE, bool NORM>
 __global__ __launch_bounds__(NT) void mid_kernel(const MidArgs a) {
     extern __shared__ __align__(16) float lt[];
     __shared__ float sm_f[NT / 64];
+    constexpr bool VEC = LIE == kPieces;
+    constexpr int G = LIE == kOne ? 1 : 4;  // elements per group
+    static_assert(LIE != kOne || (C4 == 1 && !NORM), "one element per thread");
     const int m = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int n = a.n;
     const int nmain = (n / 16) * 16;
     const float* gr = a.gate + (size_t)m * a.ldg;
     const float* ur = a.up + (size_t)m * a.ldg;
-    auto at = [&](int c, int e) { return VEC ? 4 * (c * NT + tid) + e : (4 * c + e) * NT + tid; };
+    auto at = [&](int c, int e) { return VEC ? 4 * (c * NT + tid) + e : (G * c + e) * NT + tid; };
     // (elements past the row: 0)
-    auto load4 = [&](const float* p, int c, float (&v)[4]) {
+    auto load4 = [&](const float* p, int c, float (&v)[G]) {
         if constexpr (VEC) {
             float4 x = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             if (at(c, 0) < n) x = *reinterpret_cast<const float4*>(p + at(c, 0));
@@ -483,21 +490,21 @@ __global__ __launch_bounds__(NT) void mid_kernel(const MidArgs a) {
             v[3] = x.w;
         } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = at(c, e) < n ? p[at(c, e)] : 0.0f;
+            for (int e = 0; e < G; ++e) v[e] = at(c, e) < n ? p[at(c, e)] : 0.0f;
         }
     };
-    auto store4 = [&](float* p, int c, const float (&v)[4]) {
+    auto store4 = [&](float* p, int c, const float (&v)[G]) {
         if constexpr (VEC) {
             if (at(c, 0) < n) *reinterpret_cast<float4*>(p + at(c, 0)) = make_float4(v[0], v[1], v[2], v[3]);
         } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
+            for (int e = 0; e < G; ++e)
                 if (at(c, e) < n) p[at(c, e)] = v[e];
         }
     };
-    float v[C4][4], nw[C4][4];
+    float v[C4][G], nw[C4][G];
     {
-        float g[C4][4], u[C4][4];
+        float g[C4][G], u[C4][G];
 #pragma unroll
         for (int c = 0; c < C4; ++c) {
             load4(gr, c, g[c]);
@@ -510,9 +517,9 @@ __global__ __launch_bounds__(NT) void mid_kernel(const MidArgs a) {
 #pragma unroll
         for (int c = 0; c < C4; ++c)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
+            for (int e = 0; e < G; ++e) {
                 v[c][e] = 0.0f;
-                if (!VEC && (4 * c + e) * NT >= n) continue;  // (uniform: short rows skip the code)
+                if (!VEC && (G * c + e) * NT >= n) continue;  // (uniform: short rows skip the code)
                 v[c][e] = at(c, e) < n ? apply_act(ACT, g[c][e], ACT == kActIdentity ? 0.0f : u[c][e], at(c, e) < nmain)
                                        : 0.0f;
             }
@@ -554,7 +561,7 @@ __global__ __launch_bounds__(NT) void mid_kernel(const MidArgs a) {
         for (int c = 0; c < C4; ++c) {
             if constexpr (C4 > 4) load4(a.norm_w, c, nw[c]);
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
+            for (int e = 0; e < G; ++e)
                 if (at(c, e) < n) v[c][e] = __fmul_rn(__fmul_rn(v[c][e], invr), nw[c][e]);
         }
     }
@@ -568,7 +575,7 @@ __global__ __launch_bounds__(NT) void mid_kernel(const MidArgs a) {
 #pragma unroll
     for (int c = 0; c < C4; ++c)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) mx = fmaxf(mx, fabsf(v[c][e]));
+        for (int e = 0; e < G; ++e) mx = fmaxf(mx, fabsf(v[c][e]));
     mx = wave_max_nonneg(mx);
     if (lane == 0) sm_f[w] = mx;
     __syncthreads();
@@ -583,15 +590,15 @@ __global__ __launch_bounds__(NT) void mid_kernel(const MidArgs a) {
     auto quant_row = [&](auto mode_c) {
 #pragma unroll
         for (int c = 0; c < C4; ++c) {
-            int b[4];
+            int b[G];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) b[e] = quant_one(v[c][e], scale, decltype(mode_c)::value, at(c, e) < nmain) & 255;
+            for (int e = 0; e < G; ++e) b[e] = quant_one(v[c][e], scale, decltype(mode_c)::value, at(c, e) < nmain) & 255;
             if constexpr (VEC) {
                 if (at(c, 0) < n)
                     *reinterpret_cast<int*>(qr + at(c, 0)) = b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24);
             } else {
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
+                for (int e = 0; e < G; ++e)
                     if (at(c, e) < n) qr[at(c, e)] = (int8_t)b[e];
             }
         }
@@ -604,12 +611,12 @@ __global__ __launch_bounds__(NT) void mid_kernel(const MidArgs a) {
 
 int mid_max_cols() { return 16384; }
 
-template <int NT, int C4, bool VEC, bool NORM>
+template <int NT, int C4, int LIE, bool NORM>
 static hipError_t launch_mid_t(const MidArgs& a, int M, hipStream_t s) {
     const size_t lds = NORM ? (size_t)a.n * sizeof(float) : 0;
 #define XT_MID(ACT_)                                                                          \
     case ACT_:                                                                                \
-        hipLaunchKernelGGL((mid_kernel<ACT_, NT, C4, VEC, NORM>), dim3(M), dim3(NT), lds, s, a); \
+        hipLaunchKernelGGL((mid_kernel<ACT_, NT, C4, LIE, NORM>), dim3(M), dim3(NT), lds, s, a); \
         return hipGetLastError();
     switch (a.act) {
         XT_MID(XT_ACT_RELU2_MUL)
@@ -618,7 +625,7 @@ static hipError_t launch_mid_t(const MidArgs& a, int M, hipStream_t s) {
         XT_MID(XT_ACT_SILU_MUL)
         case kActIdentity:  // (rms_norm alone)
             if constexpr (NORM) {
-                hipLaunchKernelGGL((mid_kernel<kActIdentity, NT, C4, VEC, true>), dim3(M), dim3(NT), lds, s, a);
+                hipLaunchKernelGGL((mid_kernel<kActIdentity, NT, C4, LIE, true>), dim3(M), dim3(NT), lds, s, a);
                 return hipGetLastError();
             }
     }
@@ -634,8 +641,8 @@ hipError_t launch_mlp_mid(const MidArgs& a, int M, hipStream_t s) {
                      !off(a.norm_w) && (!a.out || (a.ldo % 4 == 0 && !off(a.out))) &&
                      (!a.q || (a.ldq % 4 == 0 && ((uintptr_t)a.q & 3) == 0));
     const int n4 = (a.n + 3) / 4;
-#define XT_MIDT(NT_, C4_, VEC_, NORM_) \
-    if (n4 <= NT_ * C4_) return launch_mid_t<NT_, C4_, VEC_, NORM_>(a, M, s);
+#define XT_MIDT(NT_, C4_, LIE_, NORM_) \
+    if (n4 <= NT_ * C4_) return launch_mid_t<NT_, C4_, LIE_, NORM_>(a, M, s);
     if (a.norm_w) {
         // Measured with 256 / 512 / 1024 threads per row, us: 1 x 2560 6.4 /
         // 6.6 / 7.4, 2048 x 2560 15.8 / 20.7 / 35.8 (narrow rows overlap one
@@ -643,27 +650,34 @@ hipError_t launch_mlp_mid(const MidArgs& a, int M, hipStream_t s) {
         // 17.5, 1024 x 8640 21.7 / 24.9 / 39.2 (long rows: the blocks of 256
         // threads get long, until there are more than two rows per CU).
         if (vec && (a.n <= 4096 || M > 512)) {
-            XT_MIDT(256, 1, true, true) XT_MIDT(256, 3, true, true) XT_MIDT(256, 5, true, true)
-            XT_MIDT(256, 7, true, true) XT_MIDT(256, 9, true, true)
+            XT_MIDT(256, 1, kPieces, true) XT_MIDT(256, 3, kPieces, true) XT_MIDT(256, 5, kPieces, true)
+            XT_MIDT(256, 7, kPieces, true) XT_MIDT(256, 9, kPieces, true)
         }
-        if (vec) { XT_MIDT(512, 4, true, true) XT_MIDT(512, 8, true, true) }
-        XT_MIDT(512, 1, false, true) XT_MIDT(512, 2, false, true) XT_MIDT(512, 4, false, true)
-        XT_MIDT(512, 8, false, true)
+        if (vec) { XT_MIDT(512, 4, kPieces, true) XT_MIDT(512, 8, kPieces, true) }
+        XT_MIDT(512, 1, kSingles, true) XT_MIDT(512, 2, kSingles, true) XT_MIDT(512, 4, kSingles, true)
+        XT_MIDT(512, 8, kSingles, true)
     } else {
         // One load, one reduction: wide rows (1 x 6912 7.7 / 5.8 / 4.5 us),
-        // except where there are rows enough and a row is one piece per thread
-        // of 256 (2048 x 1024 6.3 / 7.4 / 8.3; 64 x 1024 3.5 against 2.9 with
-        // one element per thread of 1024) or more than two pieces per thread
-        // of 1024 (1024 x 8640 25.9 / 24.6 / 27.0).
-        if (a.n <= 1024 && M > 256) {
-            if (vec) { XT_MIDT(256, 1, true, false) }
-            XT_MIDT(256, 1, false, false)
+        // one element per thread where that is the row, as long as the rows
+        // leave threads idle (one element each / four: 64 x 1003 2.13 / 2.34,
+        // 300 x 64 2.03 / 2.53, 512 x 512 2.26 / 2.78, but 1024 x 1024 4.05 /
+        // 3.66 and 4096 x 512 7.7 / 7.1; rows of 256 take it at any number,
+        // 4096 x 256 3.87 / 4.45); then a piece per thread of 256 (2048 x 1024
+        // 6.3 / 7.4 / 8.3 with 256 / 512 / 1024 threads), and fewer threads
+        // again at more than two pieces per thread of 1024 (1024 x 8640 25.9 /
+        // 24.6 / 27.0).
+        if (a.n <= 256) return launch_mid_t<256, 1, kOne, false>(a, M, s);
+        if (a.n <= 512 && M <= 512) return launch_mid_t<512, 1, kOne, false>(a, M, s);
+        if (a.n <= 1024 && M <= 256) return launch_mid_t<1024, 1, kOne, false>(a, M, s);
+        if (a.n <= 1024) {
+            if (vec) { XT_MIDT(256, 1, kPieces, false) }
+            XT_MIDT(256, 1, kSingles, false)
         }
         if (vec && a.n > 1024) {
-            if (a.n > 8192 && M >= 512) { XT_MIDT(512, 5, true, false) XT_MIDT(512, 8, true, false) }
-            XT_MIDT(1024, 1, true, false) XT_MIDT(1024, 2, true, false) XT_MIDT(1024, 4, true, false)
+            if (a.n > 8192 && M >= 512) { XT_MIDT(512, 5, kPieces, false) XT_MIDT(512, 8, kPieces, false) }
+            XT_MIDT(1024, 1, kPieces, false) XT_MIDT(1024, 2, kPieces, false) XT_MIDT(1024, 4, kPieces, false)
         }
-        XT_MIDT(1024, 1, false, false) XT_MIDT(1024, 2, false, false) XT_MIDT(1024, 4, false, false)
+        XT_MIDT(1024, 1, kSingles, false) XT_MIDT(1024, 2, kSingles, false) XT_MIDT(1024, 4, kSingles, false)
     }
 #undef XT_MIDT
     return hipErrorInvalidValue;
