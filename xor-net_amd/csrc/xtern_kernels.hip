@@ -1425,7 +1425,7 @@ const GemmShape kShapes4[] = {
     {2, 8, 4, 1, 4, 2.40f, 0.338f, 0.0f, 0.294f, 0.45f, 1, 0},
     {4, 8, 4, 1, 4, 3.09f, 0.396f, 0.0f, 0.437f, 0.95f, 1, 0},
     {4, 16, 4, 1, 4, 3.82f, 0.850f, 0.0f, 0.826f, 0.82f, 1, 0},
-    {8, 16, 4, 1, 4, 4.72f, 1.673f, 0.0f, 1.316f, 1.38f, 1, 0},
+    {8, 16, 4, 1, 4, 4.65f, 1.673f, 0.0f, 1.316f, 1.38f, 1, 0},
 };
 // Pack5 (the base-3 decode is 24 vector instructions per 16 weights against
 // 9, so shapes that decode a weight once for 128 tokens pay earlier): 3200 ->
