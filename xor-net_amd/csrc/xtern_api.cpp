@@ -315,8 +315,10 @@ int run_product(const xt_weights* const* ws, int n, const int8_t* q, int ldq, co
     a.nch = (int)ws[0]->nch;
     a.cps = (a.nch + cfg.splitk - 1) / cfg.splitk;
     const int64_t gy = (M + 16 * cfg.mb - 1) / (16 * cfg.mb);
-    // (rows per launch: 65535 blocks of 32 tokens up to 18 Pack4 or 8 Pack5
-    // chunks of K, of 16 tokens beyond)
+    // Rows per call: 65535 blocks of 32 tokens up to 18 Pack4 or 8 Pack5 chunks
+    // of K, of 16 tokens beyond.  (The interface's limit, settled by the
+    // launches of earlier kernels: gemmw_kernel has no row blocks in y and
+    // would take more; mm_kernel's are its grid's y.)
     const int64_t block = a.nch <= (fmt == XT_PACK5 ? 8 : 18) ? 32 : 16;
     if (M > 65535 * block || (cfg.kind != 4 && gy > 65535)) return fail(XT_ERR_UNSUPPORTED, "M too large for one launch");
     if (cfg.kind == 2) {
@@ -471,6 +473,8 @@ int linear_f32(const xt_weights* const* ws, int n, const float* x, int64_t M, fl
     const size_t qbytes = align_up((size_t)M * kpad, 256);
     const size_t fbytes = align_up((size_t)M * 4, 256);
     void* wsp = nullptr;
+    // (the second vector is spare: which rows the fixed scratch of the
+    // allocation-free call takes was settled with row sums in it)
     if (int rc = workspace(s, qbytes + 2 * fbytes, &wsp, 0, sc)) return rc;
     int8_t* q = static_cast<int8_t*>(wsp);
     float* inv = reinterpret_cast<float*>(static_cast<char*>(wsp) + qbytes);

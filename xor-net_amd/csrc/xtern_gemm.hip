@@ -87,7 +87,8 @@ typedef const __attribute__((address_space(4))) MMArgs* KArgPtr;
 // its 32 NW rows (MW x NW accumulator blocks of 32 x 32).
 //
 // What bounds it: on long prompts the matrix cores at the clock they are left
-// (about 1.95 GHz under this load; 61 % of the cycles have an MFMA in flight),
+// (1.8 to 1.95 GHz under this load; 60 to 66 % of the cycles have an MFMA in
+// flight, by the counter that the cycles are taken from),
 // on shapes of one workgroup per CU the issue of one wave per SIMD: 9 (Pack5
 // 24) decode instructions per weight block and k-step next to 32 cycles per
 // MFMA.  So:
@@ -110,7 +111,7 @@ typedef const __attribute__((address_space(4))) MMArgs* KArgPtr;
 //    next chunk and starts the loads of chunk c + D.
 // The kernels it replaced (32 x 128 and 16 x 80 tiles) decoded every weight
 // for 16 or 32 tokens only.  Measured, launch to launch: M = 4096, 4096 ->
-// 14336 1094 -> 203 us (2.37 POP/s), M = 512, 2560 -> 13824 45 -> 21, 6912 ->
+// 14336 1094 -> 194 us (2.48 POP/s), M = 512, 2560 -> 13824 45 -> 21, 6912 ->
 // 2560 32 -> 16; Pack5 M = 1024, 3200 -> 17280 226 -> 74, 8640 -> 3200 92 ->
 // 37.  Two groups of waves taking alternate chunks (more waves per SIMD), and
 // starting the workgroups that share operands at different chunks, changed
@@ -202,7 +203,7 @@ __global__ __launch_bounds__(64 * W, 2) void gemmw_kernel(const MMArgs a) {
 #pragma unroll
         for (int nb = 0; nb < NW; ++nb)
 #pragma unroll
-            for (int L = 0; L < 2; ++L) 
+            for (int L = 0; L < 2; ++L)
                 w[nb][L] = __builtin_amdgcn_raw_buffer_load_b128(wbuf, (int)woff[nb] + 512 * L, (int)off, 0);
     };
     const unsigned fr = FMT == XT_PACK5 ? (unsigned)(r * CH) : (unsigned)(r * CH + 16 * (h ^ (r & 15)));
