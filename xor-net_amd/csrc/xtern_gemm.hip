@@ -204,7 +204,7 @@ __global__ __launch_bounds__(64 * W, 2) void gemmw_kernel(const MMArgs a) {
         for (int nb = 0; nb < NW; ++nb)
 #pragma unroll
             for (int L = 0; L < 2; ++L)
-                w[nb][L] = __builtin_amdgcn_raw_buffer_load_b128(wbuf, (int)woff[nb] + 512 * L, (int)off, 0);
+                w[nb][L] = __builtin_amdgcn_raw_buffer_load_b128(wbuf, (int)(woff[nb] + 512u * L), (int)off, 0);
     };
     const unsigned fr = FMT == XT_PACK5 ? (unsigned)(r * CH) : (unsigned)(r * CH + 16 * (h ^ (r & 15)));
     auto read_f = [&](const uint8_t* src, int L, int s, v4i (&av)[MW]) {
