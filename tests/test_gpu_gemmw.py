@@ -1,5 +1,5 @@
-"""The many-row GEMM (gemmw_kernel) in every compiled shape, forced one at a
-time: chunk counts around its buffer counts (2, 3, 4: whole rounds, every
+"""The many-row GEMM (gemmw_kernel) in every compiled shape, and the 16-token
+shapes (mm_kernel) that the same rule chooses from, forced one at a time: chunk counts around its buffer counts (2, 3, 4: whole rounds, every
 remainder, fewer chunks than buffers), token and output-row remainders, ragged
 K, projections that end inside a tile, i32 accumulators requested or not.
 Integer sums and two f32 roundings: everything is compared bit for bit."""
@@ -73,6 +73,32 @@ def test_forced_shapes_several_projections(fmt, shape, monkeypatch):
         ys = xtern.linear_multi_q([w for _, w in made], torch.from_numpy(q).to(DEV), torch.from_numpy(inv).to(DEV))
         for (t, _), s, y in zip(made, scales, ys):
             assert np.array_equal(y.cpu().numpy().view(np.int32), reference(t, q, inv, s)[1])
+
+
+@pytest.mark.parametrize("fmt,shape", [(xtern.XT_PACK4, s) for s in ("1,2,4,4,1", "1,4,8,2,1", "1,5,8,2,1", "1,8,8,2,1")]
+                         + [(xtern.XT_XORSPARSE, "1,2,4,4,1")]
+                         + [(xtern.XT_PACK5, s) for s in ("1,2,4,4,1", "1,4,8,2,1", "1,5,8,2,1", "1,5,16,1,1")])
+def test_sixteen_token_shapes_exact(fmt, shape, monkeypatch):
+    """Rows multiplied as they are (whole chunks, aligned: the kernel sums them
+    itself) and through the padded copy (ragged K, or rows off 16 bytes: their
+    sums are given), fewer and more chunks than a round of the waves, one and
+    several projections."""
+    monkeypatch.setenv("XTERN_CONFIG", shape)
+    rng = np.random.default_rng(13)
+    ch = 320 if fmt == xtern.XT_PACK5 else 256
+    for M, K, widths in ((17, ch, (16,)), (33, 4 * ch, (129, 31)), (160, 9 * ch, (700,)), (48, 17 * ch, (96, 33, 257)),
+                         (40, 5 * ch - 4, (130,)), (65, 18 * ch + 20, (33, 640))):
+        print(f"[case] {shape} fmt={fmt} M={M} K={K} N={widths}", flush=True)
+        q = rng.integers(-128, 128, (M, K)).astype(np.int8)
+        inv = rng.uniform(1e-3, 0.1, M).astype(np.float32)
+        scales = [rng.uniform(0.2, 2.0, N).astype(np.float32) for N in widths]
+        made = [weights(rng, fmt, K, N, s) for N, s in zip(widths, scales)]
+        off = torch.empty(M * K + 4, dtype=torch.int8, device=DEV)[4:].view(M, K)
+        off.copy_(torch.from_numpy(q))
+        for qd in (torch.from_numpy(q).to(DEV), off):
+            ys = xtern.linear_multi_q([w for _, w in made], qd, torch.from_numpy(inv).to(DEV))
+            for (t, _), s, y in zip(made, scales, ys):
+                assert np.array_equal(y.cpu().numpy().view(np.int32), reference(t, q, inv, s)[1])
 
 
 @pytest.mark.parametrize("fmt", [xtern.XT_PACK4, xtern.XT_PACK5], ids=["pack4", "pack5"])
